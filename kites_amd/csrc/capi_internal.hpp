@@ -43,6 +43,9 @@ struct kites_graph {
   kites::device_buffer<unsigned> levels;
   uint32_t bfs_k = 0;
   std::vector<kites::detail::bitbfs_stats> bfs_stats;
+  // PageRank: values (n) and edge weights (m), and the ordered runs' state.
+  kites::device_buffer<float> pr;
+  kites::detail::ordered_workspace pr_ws;
 };
 
 namespace kites_capi {

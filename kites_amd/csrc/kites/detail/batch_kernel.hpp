@@ -96,17 +96,6 @@ struct batch_params {
   batch_params(FN f) : fn(f) {}
 };
 
-__device__ __forceinline__ unsigned wave_incl_max(unsigned x) {
-  unsigned y;
-  y = dpp<0x111>(x); x = x > y ? x : y;
-  y = dpp<0x112>(x); x = x > y ? x : y;
-  y = dpp<0x114>(x); x = x > y ? x : y;
-  y = dpp<0x118>(x); x = x > y ? x : y;
-  y = dpp<0x142, 0xa>(x); x = x > y ? x : y;
-  y = dpp<0x143, 0xc>(x); x = x > y ? x : y;
-  return x;
-}
-
 __device__ __forceinline__ unsigned long long readlane64(unsigned long long x, unsigned lane) {
   unsigned const lo = __builtin_amdgcn_readlane(static_cast<unsigned>(x), lane);
   unsigned const hi = __builtin_amdgcn_readlane(static_cast<unsigned>(x >> 32), lane);

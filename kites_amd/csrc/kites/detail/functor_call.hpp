@@ -1,0 +1,92 @@
+// functor_call.hpp -- how the kernels call the four functors.
+//
+// The reference's signatures take volatile references (README.md:16-23).  A
+// volatile access through a reference stays a flat access with system scope
+// (flat_load / flat_store sc0 sc1) even when it points into LDS, and the wave
+// then waits for every load it has in flight.  Functors that take plain
+// references instead ("vT&" where the reference has "volatile vT&"; the
+// library's own sets do) work on registers.  Which form a functor has is seen
+// from its signature: a plain reference does not bind to a volatile lvalue.
+//
+// The *_at forms work on LDS slots in place; edge_value returns the partial.
+#ifndef KITES_DETAIL_FUNCTOR_CALL_HPP_
+#define KITES_DETAIL_FUNCTOR_CALL_HPP_
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+namespace kites {
+namespace detail {
+
+template <class T>
+__host__ __device__ __forceinline__ volatile T& as_volatile(T& x) {
+  return *reinterpret_cast<volatile T*>(&x);
+}
+
+// nbrCompF(partial, srcV, edge); `slot`: an LDS slot of the calling lane.
+template <class FN, class vT, class eT>
+__device__ __forceinline__ vT edge_value(FN& fn, vT& slot, vT src, eT* edge) {
+  if constexpr (std::is_invocable<FN&, volatile vT&, vT, eT*>::value) {
+    fn(as_volatile(slot), src, edge);
+    return slot;
+  } else {
+    vT r{};
+    fn(r, src, edge);
+    return r;
+  }
+}
+
+template <class FN, class vT, class eT>
+__device__ __forceinline__ void edge_value_at(FN& fn, vT& slot, vT src, eT* edge) {
+  if constexpr (std::is_invocable<FN&, volatile vT&, vT, eT*>::value) {
+    fn(as_volatile(slot), src, edge);
+  } else {
+    vT r{};
+    fn(r, src, edge);
+    slot = r;
+  }
+}
+
+// initF(local, global)
+template <class FI, class vT>
+__device__ __forceinline__ void init_at(FI& fi, vT& slot, vT global) {
+  vT g = global;
+  if constexpr (std::is_invocable<FI&, volatile vT&, vT&>::value) {
+    fi(as_volatile(slot), g);
+  } else {
+    vT r{};
+    fi(r, g);
+    slot = r;
+  }
+}
+
+// redF(lhs, rhs)
+template <class FR, class vT>
+__device__ __forceinline__ void reduce_at(FR& fr, vT& lhs, vT& rhs) {
+  if constexpr (std::is_invocable<FR&, volatile vT&, volatile vT&>::value) {
+    fr(as_volatile(lhs), as_volatile(rhs));
+  } else {
+    vT l = lhs, r = rhs;
+    fr(l, r);
+    lhs = l;
+  }
+}
+
+// updF(newV, oldV)
+template <class FU, class vT>
+__device__ __forceinline__ bool update_at(FU& fu, vT& slot, vT old) {
+  if constexpr (std::is_invocable<FU&, volatile vT&, vT>::value) {
+    return fu(as_volatile(slot), old);
+  } else {
+    vT nv = slot;
+    bool const u = fu(nv, old);
+    slot = nv;
+    return u;
+  }
+}
+
+}  // namespace detail
+}  // namespace kites
+
+#endif  // KITES_DETAIL_FUNCTOR_CALL_HPP_

@@ -59,6 +59,18 @@ __device__ __forceinline__ unsigned wave_incl_scan(unsigned x) {
   return x;
 }
 
+// Inclusive prefix maximum over the 64 lanes (u32).
+__device__ __forceinline__ unsigned wave_incl_max(unsigned x) {
+  unsigned y;
+  y = dpp<0x111>(x); x = x > y ? x : y;
+  y = dpp<0x112>(x); x = x > y ? x : y;
+  y = dpp<0x114>(x); x = x > y ? x : y;
+  y = dpp<0x118>(x); x = x > y ? x : y;
+  y = dpp<0x142, 0xa>(x); x = x > y ? x : y;
+  y = dpp<0x143, 0xc>(x); x = x > y ? x : y;
+  return x;
+}
+
 __device__ __forceinline__ unsigned wave_sum(unsigned x) {
   return readlane(wave_incl_scan(x), 63);
 }

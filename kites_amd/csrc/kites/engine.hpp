@@ -525,73 +525,107 @@ unsigned record_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options c
 
 namespace detail {
 
-// The ordered mode's loop: per iteration, copy the values, clear the next
-// frontier and the flag, run ordered_kernel, read the flag; the values and
-// the frontiers alternate between two buffers.
-template <class vT, class eT, class vIdxT, class FI, class FN, class FR, class FU>
-void run_ordered(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, stream& s, workspace& ws,
-                 FI fi, FN fn, FR fr, FU fu, options const& o) {
-  std::size_t const n = grph.get_num_vertices();
-  int const did = grph.getResidingDeviceID();
-  device_buffer<vT> vb(n ? n : 1, did);
-  unsigned long long* const bm0 = ws.bm.get_ptr();
-  unsigned long long* const bm1 = bm0 + ws.nwords;
-  std::size_t const wbytes = static_cast<std::size_t>(ws.nwords) * sizeof(unsigned long long);
-  KITES_HIP_CHECK(hipEventRecord(ws.ev0, s.get()));
-  KITES_HIP_CHECK(hipMemsetAsync(bm0, 0, 2 * wbytes, s.get()));
-  // the initial frontier is consumed, as in the other schedules
-  std::size_t const fb = std::min<std::size_t>(grph.vBitmapEven.sizeInBytes(), wbytes);
-  if (fb) {
-    KITES_HIP_CHECK(hipMemcpyAsync(bm0, grph.vBitmapEven.get_ptr(), fb, hipMemcpyDeviceToDevice,
-                                   s.get()));
-    KITES_HIP_CHECK(hipMemsetAsync(grph.vBitmapEven.get_ptr(), 0, grph.vBitmapEven.sizeInBytes(),
-                                   s.get()));
-  }
+// The graph arrays an ordered run reads.
+template <class vT, class eT>
+struct ordered_view {
+  std::size_t n, m;
+  const unsigned *R, *C;
+  eT* E;
+  const unsigned *oR, *oC, *nzi, *nzR;
+  unsigned nnz;
+  vT* V;                              // values in and out
+  const unsigned long long* frontier; // initial active vertices (null: all)
+  std::size_t frontier_bytes;
+};
+
+// The ordered mode's loop over the view `g` (detail/ordered_kernel.hpp): two
+// launches per iteration, the iteration index, the activity form and the done
+// flag on the device; the host queues kOrderedChunk iterations and then reads
+// the control header once.
+constexpr unsigned kOrderedChunk = 4;
+
+template <class vT, class eT, class FI, class FN, class FR, class FU>
+void run_ordered(ordered_view<vT, eT> const& g, gpu& dev, stream& s, ordered_workspace& ws, FI fi,
+                 FN fn, FR fr, FU fu, options const& o) {
+  using S = ordered_shape<vT>;
   using P = ordered_params<vT, eT, FI, FN, FR, FU>;
+  std::size_t const n = g.n, m = g.m;
+  unsigned const nwords = static_cast<unsigned>((n + 63) / 64 + 1);
+  unsigned const ntasks = static_cast<unsigned>(m / S::task_edges + 1);
+  // a heavy vertex holds more than S::light in-edges
+  std::size_t const hcap = m / (S::light + 1) + 1, ccap = m / 64 + hcap + 1;
   param_block<P> pb(fi, fn, fr, fu);
   P& prm = pb.get();
   prm.n = static_cast<unsigned>(n);
-  prm.R = reinterpret_cast<const unsigned*>(grph.R.get_ptr());
-  prm.C = reinterpret_cast<const unsigned*>(grph.C.get_ptr());
-  prm.E = grph.E.get_ptr();
-  prm.oR = reinterpret_cast<const unsigned*>(grph.oR.get_ptr());
-  prm.oC = reinterpret_cast<const unsigned*>(grph.oC.get_ptr());
-  prm.nwords = ws.nwords;
-  prm.flag = grph.updateFlag.get_ptr();
-  vT* vin = grph.V.get_ptr();
-  vT* vout = vb.get_ptr();
-  unsigned long long* bin = bm0;
-  unsigned long long* bout = bm1;
-  unsigned const grid = static_cast<unsigned>(dev.numComputeUnits()) * 8u;
+  prm.m = m;
+  prm.R = g.R;
+  prm.C = g.C;
+  prm.E = g.E;
+  prm.oR = g.oR;
+  prm.oC = g.oC;
+  prm.nzi = g.nzi;
+  prm.nzR = g.nzR;
+  prm.nnz = g.nnz;
+  prm.V = g.V;
+  prm.nwords = nwords;
+  prm.ntasks = ntasks;
+  ws.begin();
+  ws.add(prm.W, n);
+  ws.add(prm.bm, 2 * static_cast<std::size_t>(nwords));
+  ws.add(prm.hasin, nwords);
+  ws.add(prm.tstart, static_cast<std::size_t>(ntasks) + 1);
+  ws.add(prm.hv, hcap);
+  ws.add(prm.hbase, hcap);
+  ws.add(prm.hact, hcap);
+  ws.add(prm.hchunk, ccap);
+  ws.add(prm.hsum, ccap);
+  ws.add(prm.ctl, 1);
+  ws.commit(dev.getDevIdx());
+  KITES_HIP_CHECK(hipEventRecord(ws.ev0, s.get()));
   unsigned const max_iter = std::max(1u, o.max_iterations);
-  unsigned iters = 0;
-  bool done = false;
-  while (iters < max_iter) {
-    if (n)
-      KITES_HIP_CHECK(hipMemcpyAsync(vout, vin, n * sizeof(vT), hipMemcpyDeviceToDevice, s.get()));
-    KITES_HIP_CHECK(hipMemsetAsync(bout, 0, wbytes, s.get()));
-    KITES_HIP_CHECK(hipMemsetAsync(prm.flag, 0, sizeof(unsigned), s.get()));
-    prm.Vin = vin;
-    prm.Vout = vout;
-    prm.in_bm = bin;
-    prm.out_bm = bout;
-    auto const kern = &ordered_kernel<256, P>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s.get(), prm);
+  unsigned const cus = static_cast<unsigned>(dev.numComputeUnits());
+  auto blocks = [&](std::size_t items, std::size_t per) {
+    return static_cast<unsigned>(
+        std::min<std::size_t>(std::max<std::size_t>((items + per - 1) / per, 1), cus * 8u));
+  };
+  hipLaunchKernelGGL(ordered_reset_kernel, dim3(1), dim3(128), 0, s.get(), prm.ctl, max_iter,
+                     g.frontier ? 0u : 1u);
+  hipLaunchKernelGGL(ordered_vertices_kernel<S::light>, dim3(blocks(nwords, 4)), dim3(256), 0,
+                     s.get(), prm.R, prm.n, nwords, prm.hasin, prm.hv, prm.hbase, prm.hact,
+                     prm.ctl);
+  hipLaunchKernelGGL(ordered_tasks_kernel<S::task_edges>, dim3(blocks(ntasks, 256)), dim3(256), 0,
+                     s.get(), prm.R, prm.nzR, prm.nnz, ntasks, prm.tstart, prm.hv, prm.hbase,
+                     prm.hchunk, prm.ctl);
+  hipLaunchKernelGGL(ordered_frontier_kernel, dim3(blocks(nwords, 256)), dim3(256), 0, s.get(),
+                     g.frontier,
+                     static_cast<unsigned>(std::min<std::size_t>(g.frontier_bytes / 8, nwords)),
+                     prm.n, nwords, prm.bm);
+  KITES_HIP_CHECK(hipPeekAtLastError());
+  auto const heavy = &ordered_heavy_kernel<P>;
+  auto const kern = &ordered_kernel<P>;
+  unsigned const hgrid =
+      blocks(std::max<std::size_t>(n / 4, m / (16 * S::heavy_unroll)), S::block);
+  unsigned const mgrid = blocks(std::max<std::size_t>(ntasks, nwords), S::waves);
+  unsigned long long launched = 0;
+  for (;;) {
+    for (unsigned k = 0; k < kOrderedChunk; ++k) {
+      hipLaunchKernelGGL(heavy, dim3(hgrid), dim3(S::block), 0, s.get(), prm);
+      hipLaunchKernelGGL(kern, dim3(mgrid), dim3(S::block), 0, s.get(), prm);
+    }
     KITES_HIP_CHECK(hipPeekAtLastError());
-    KITES_HIP_CHECK(hipMemcpyAsync(grph.updateFlagHost.get_ptr(), prm.flag, sizeof(unsigned),
+    launched += kOrderedChunk;
+    KITES_HIP_CHECK(hipMemcpyAsync(ws.host.get_ptr(), prm.ctl, offsetof(ordered_ctl, slots),
                                    hipMemcpyDeviceToHost, s.get()));
     s.sync();
-    ++iters;
-    std::swap(vin, vout);
-    std::swap(bin, bout);
-    if (grph.updateFlagHost[0] == 0) {
-      done = true;
+    if (ws.host[0].done || launched > static_cast<unsigned long long>(max_iter) + kOrderedChunk)
       break;
-    }
   }
-  if (vin != grph.V.get_ptr() && n)
-    KITES_HIP_CHECK(hipMemcpyAsync(grph.V.get_ptr(), vin, n * sizeof(vT), hipMemcpyDeviceToDevice,
-                                   s.get()));
+  // (at convergence both buffers hold the result: the last iteration moved
+  // nothing)
+  unsigned const iters = ws.host[0].iter;
+  bool const done = ws.host[0].done == 1;
+  if (!done && (iters & 1) && n)
+    KITES_HIP_CHECK(hipMemcpyAsync(g.V, prm.W, n * sizeof(vT), hipMemcpyDeviceToDevice, s.get()));
   KITES_HIP_CHECK(hipEventRecord(ws.ev1, s.get()));
   s.sync();
   float ms = 0.f;
@@ -607,6 +641,39 @@ void run_ordered(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, stream& s, wor
     o.report->delta = false;
     o.report->min_fast = false;
   }
+}
+
+// The ordered mode on a device graph; the initial frontier is consumed, as in
+// the other schedules.
+template <class vT, class eT, class vIdxT, class FI, class FN, class FR, class FU>
+void run_ordered_graph(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, stream& s, workspace& ws,
+                       FI fi, FN fn, FR fr, FU fu, options const& o) {
+  ordered_view<vT, eT> g;
+  g.n = grph.get_num_vertices();
+  g.m = grph.get_num_edges();
+  g.R = reinterpret_cast<const unsigned*>(grph.R.get_ptr());
+  g.C = reinterpret_cast<const unsigned*>(grph.C.get_ptr());
+  g.E = grph.E.get_ptr();
+  g.oR = reinterpret_cast<const unsigned*>(grph.oR.get_ptr());
+  g.oC = reinterpret_cast<const unsigned*>(grph.oC.get_ptr());
+  g.nzi = reinterpret_cast<const unsigned*>(grph.nzi.get_ptr());
+  g.nzR = reinterpret_cast<const unsigned*>(grph.nzR.get_ptr());
+  g.nnz = grph.nnz;
+  g.V = grph.V.get_ptr();
+  // (a graph of an explicit frontier bitmap; an empty one activates nothing)
+  g.frontier = grph.vBitmapEven.get_ptr();
+  g.frontier_bytes = grph.vBitmapEven.sizeInBytes();
+  if (g.nnz == 0 && g.m != 0)
+    throw std::runtime_error("kites::process: the ordered mode needs the graph's in-edge list");
+  try {
+    run_ordered(g, dev, s, ws.ord, fi, fn, fr, fu, o);
+  } catch (...) {
+    (void)hipMemsetAsync(grph.vBitmapEven.get_ptr(), 0, grph.vBitmapEven.sizeInBytes(), s.get());
+    throw;
+  }
+  if (g.frontier_bytes)
+    KITES_HIP_CHECK(hipMemsetAsync(grph.vBitmapEven.get_ptr(), 0, g.frontier_bytes, s.get()));
+  s.sync();
 }
 
 }  // namespace detail
@@ -652,7 +719,7 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
         "workspace");
   if (o.ordered) {
     if (vpg != 1) throw std::runtime_error("kites::process: the ordered mode needs vertex-per-group 1");
-    run_ordered(grph, dev, s, *ws, funcInit, funcCompNbr, funcRed, funcUpd, o);
+    run_ordered_graph(grph, dev, s, *ws, funcInit, funcCompNbr, funcRed, funcUpd, o);
     return;
   }
   probe_result const pr = probe_functors<vT, eT>(funcInit, funcCompNbr, funcRed, funcUpd);
@@ -861,8 +928,9 @@ void process(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcInit
   }
   if (!grph.ws) grph.ws.reset(new workspace());
   workspace& ws = *grph.ws;
-  ws.ensure(n, std::max(2u, o.max_iterations), grph.getResidingDeviceID());
-  if (o.delta) ws.ensure_far();
+  // (an ordered run keeps its state in ws.ord)
+  if (!o.ordered) ws.ensure(n, std::max(2u, o.max_iterations), grph.getResidingDeviceID());
+  if (o.delta && !o.ordered) ws.ensure_far();
   run_state st = state_of(ws);
   run_engine(grph, dev, funcInit, funcCompNbr, funcRed, funcUpd, o, st, &ws);
 }

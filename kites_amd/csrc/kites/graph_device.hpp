@@ -23,12 +23,14 @@
 #include <chrono>
 #include <iostream>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "common.hpp"
 #include "detail/batch_kernel.hpp"
 #include "detail/bitbfs_kernel.hpp"
 #include "detail/launch_cache.hpp"
+#include "detail/ordered_kernel.hpp"
 #include "detail/step_kernel.hpp"
 #include "device.hpp"
 #include "graph.hpp"
@@ -66,6 +68,40 @@ struct batch_workspace {
   }
 };
 
+// Device state of ordered runs: one allocation, kept between runs and grown
+// when a run needs more, cut into the run's arrays (add() each, then commit()).
+struct ordered_workspace {
+  device_buffer<unsigned char> mem;
+  host_pinned_buffer<ordered_ctl> host;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  std::vector<std::pair<unsigned char**, std::size_t>> parts;
+  std::size_t bytes = 0;
+
+  void begin() {
+    parts.clear();
+    bytes = 0;
+  }
+  template <class T>
+  void add(T*& p, std::size_t count) {
+    parts.emplace_back(reinterpret_cast<unsigned char**>(&p), bytes);
+    bytes += (count * sizeof(T) + 255) & ~std::size_t(255);
+  }
+  void commit(int dev) {
+    if (mem.size() < bytes) {
+      mem.free();
+      mem.alloc(bytes, dev);
+    }
+    if (host.size() == 0) host.alloc(1);
+    if (!ev0) KITES_HIP_CHECK(hipEventCreate(&ev0));
+    if (!ev1) KITES_HIP_CHECK(hipEventCreate(&ev1));
+    for (auto const& x : parts) *x.first = mem.get_ptr() + x.second;
+  }
+  ~ordered_workspace() {
+    if (ev0) (void)hipEventDestroy(ev0);
+    if (ev1) (void)hipEventDestroy(ev1);
+  }
+};
+
 // Per-run scratch of the engine (one per device graph).
 struct workspace {
   int dev = 0;
@@ -81,6 +117,7 @@ struct workspace {
   device_buffer<step_ctl> ctl;
   host_pinned_buffer<step_ctl> ctl_host;
   device_buffer<group_stats> gst;         // per-group partial statistics
+  ordered_workspace ord;                   // ordered runs (allocated by the first one)
   launch_cache graphs;                     // captured iteration chunks
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the two control-line copies in flight

@@ -19,14 +19,9 @@ static __global__ void inv_outdeg_kernel(const unsigned* __restrict__ oR,
   }
 }
 
-static __global__ void fill_kernel(float* __restrict__ V, unsigned n, float x,
-                                   unsigned long long* __restrict__ bits, unsigned words) {
+static __global__ void fill_kernel(float* __restrict__ V, unsigned n, float x) {
   unsigned const stride = gridDim.x * blockDim.x;
   for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) V[i] = x;
-  for (unsigned w = blockIdx.x * blockDim.x + threadIdx.x; w < words; w += stride) {
-    unsigned const lo = w * 64u;
-    bits[w] = lo >= n ? 0ull : (n - lo >= 64 ? ~0ull : ((1ull << (n - lo)) - 1ull));
-  }
 }
 
 }  // namespace
@@ -44,43 +39,55 @@ int kites_pagerank_f32(kites_graph* g, float damping, float tol, uint32_t max_it
   int const did = dev.getDevIdx();
   std::size_t const n = g->n;
   std::size_t const m = g->m;
-  // A float view of the graph: the same in-CSR and out-lists, weights
-  // 1 / outdeg(source).
-  kites::graph_csr_device<float, float> f(n, dev);
+  // The float values and the weights 1 / outdeg(source) in the handle's
+  // PageRank buffer; the graph's arrays are read where they are.
   kites::stream& s = dev.getSsEven();
-  auto d2d = [&](void* d, const void* h, std::size_t bytes) {
-    if (bytes) KITES_HIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyDeviceToDevice, s.get()));
-  };
-  f.C.alloc(m ? m : 1, did);
-  f.E.alloc(m ? m : 1, did);
-  f.oC.alloc(m ? m : 1, did);
-  d2d(f.R.get_ptr(), src.R.get_ptr(), (n + 1) * 4);
-  d2d(f.C.get_ptr(), src.C.get_ptr(), m * 4);
-  d2d(f.oR.get_ptr(), src.oR.get_ptr(), (n + 1) * 4);
-  d2d(f.oC.get_ptr(), src.oC.get_ptr(), m * 4);
-  f.set_num_edges(m);
+  dev.setAsActive();
+  if (g->pr.size() < n + m) {
+    g->pr.free();
+    g->pr.alloc(n + m, did);
+  }
+  float* const V = g->pr.get_ptr();
+  float* const W = V + n;
   unsigned const cus = static_cast<unsigned>(dev.numComputeUnits());
   if (m)
     hipLaunchKernelGGL(inv_outdeg_kernel, dim3(cus * 8), dim3(256), 0, s.get(),
                        reinterpret_cast<const unsigned*>(src.oR.get_ptr()),
                        reinterpret_cast<const unsigned*>(src.C.get_ptr()),
-                       static_cast<unsigned>(m), f.E.get_ptr());
+                       static_cast<unsigned>(m), W);
   // every vertex starts at 1 and active
-  hipLaunchKernelGGL(fill_kernel, dim3(cus * 8), dim3(256), 0, s.get(), f.V.get_ptr(),
-                     static_cast<unsigned>(n), 1.0f, f.vBitmapEven.get_ptr(),
-                     static_cast<unsigned>(f.vBitmapEven.size()));
+  hipLaunchKernelGGL(fill_kernel, dim3(cus * 8), dim3(256), 0, s.get(), V,
+                     static_cast<unsigned>(n), 1.0f);
   KITES_HIP_CHECK(hipPeekAtLastError());
-  s.sync();
+  kites::detail::ordered_view<float, float> f;
+  f.n = n;
+  f.m = m;
+  f.R = src.R.get_ptr();
+  f.C = src.C.get_ptr();
+  f.E = W;
+  f.oR = src.oR.get_ptr();
+  f.oC = src.oC.get_ptr();
+  f.nzi = src.nzi.get_ptr();
+  f.nzR = src.nzR.get_ptr();
+  f.nnz = src.nnz;
+  f.V = V;
+  f.frontier = nullptr;
+  f.frontier_bytes = 0;
 
+  // Plain-reference functors (operands in registers); no contraction: a
+  // product and a sum each round on their own, as the combine order defines.
   float const base = 1.0f - damping;
-  auto initF = [base] __host__ __device__(volatile float& locV, float&) { locV = base; };
-  auto nbrF = [damping] __host__ __device__(volatile float& partialV, float srcV, float* connE) {
+  auto initF = [base] __host__ __device__(float& locV, float&) { locV = base; };
+  auto nbrF = [damping] __host__ __device__(float& partialV, float srcV, float* connE) {
+#pragma clang fp contract(off)
     partialV = damping * srcV * (*connE);
   };
-  auto redF = [] __host__ __device__(volatile float& lhsV, volatile float& rhsV) {
+  auto redF = [] __host__ __device__(float& lhsV, float& rhsV) {
+#pragma clang fp contract(off)
     lhsV = lhsV + rhsV;
   };
-  auto updF = [tol] __host__ __device__(volatile float& newV, float oldV) {
+  auto updF = [tol] __host__ __device__(float& newV, float oldV) {
+#pragma clang fp contract(off)
     float const d = newV - oldV;
     return d > tol || d < -tol;
   };
@@ -89,9 +96,9 @@ int kites_pagerank_f32(kites_graph* g, float damping, float tol, uint32_t max_it
   o.ordered = true;
   o.max_iterations = max_iterations ? max_iterations : 10000u;
   o.report = &rep;
-  kites::process<kites::launch::sync>(f, dev, initF, nbrF, redF, updF, o);
+  kites::detail::run_ordered(f, dev, s, g->pr_ws, initF, nbrF, redF, updF, o);
   if (out && n)
-    KITES_HIP_CHECK(hipMemcpy(out, f.V.get_ptr(), n * sizeof(float), hipMemcpyDeviceToHost));
+    KITES_HIP_CHECK(hipMemcpy(out, V, n * sizeof(float), hipMemcpyDeviceToHost));
   if (info) {
     info->iterations = rep.iterations;
     info->ms = static_cast<float>(rep.ms);
