@@ -167,7 +167,9 @@ struct workspace {
       ctl.alloc(1, dev);
       ctl_host.alloc(2);
       gst.alloc(kTicketGroups, dev);
-      KITES_HIP_CHECK(hipMemset(ctl.get_ptr(), 0, sizeof(step_ctl)));
+      // (reset_kernel writes all of the control block that a run reads, on the
+      // run's own stream; a null-stream memset here would not be ordered
+      // before it, the stream being a non-blocking one)
       KITES_HIP_CHECK(hipEventCreate(&ev0));
       KITES_HIP_CHECK(hipEventCreate(&ev1));
       KITES_HIP_CHECK(hipEventCreateWithFlags(&evc[0], hipEventDisableTiming));
