@@ -15,14 +15,14 @@ template <class Body>
 void with_min_functors(int algo, Body&& body) {
   using vT = unsigned;
   using eT = unsigned;
-  auto initF = [] __host__ __device__(volatile vT& locV, vT& globV) { locV = globV; };
-  auto redMin = [] __host__ __device__(volatile vT& lhsV, volatile vT& rhsV) {
+  auto initF = [] __host__ __device__(vT& locV, vT& globV) { locV = globV; };
+  auto redMin = [] __host__ __device__(vT& lhsV, vT& rhsV) {
     if (lhsV > rhsV) lhsV = rhsV;
   };
-  auto updLess = [] __host__ __device__(volatile vT& newV, vT oldV) { return newV < oldV; };
+  auto updLess = [] __host__ __device__(vT& newV, vT oldV) { return newV < oldV; };
   switch (algo) {
     case KITES_ALGO_SSSP: {
-      auto nbr = [] __host__ __device__(volatile vT& partialV, vT srcV, eT* connE) {
+      auto nbr = [] __host__ __device__(vT& partialV, vT srcV, eT* connE) {
         vT const t = srcV + *connE;
         partialV = (srcV == 0xFFFFFFFFu || t < srcV) ? 0xFFFFFFFFu : t;
       };
@@ -30,7 +30,7 @@ void with_min_functors(int algo, Body&& body) {
       break;
     }
     case KITES_ALGO_BFS: {
-      auto nbr = [] __host__ __device__(volatile vT& partialV, vT srcV, eT*) {
+      auto nbr = [] __host__ __device__(vT& partialV, vT srcV, eT*) {
         partialV = (srcV == 0xFFFFFFFFu) ? 0xFFFFFFFFu : srcV + 1u;
       };
       body(initF, nbr, redMin, updLess);

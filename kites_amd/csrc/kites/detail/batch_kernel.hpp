@@ -322,8 +322,7 @@ __global__ __launch_bounds__(BLOCK) void batch_step_kernel(P p) {
               oldv = p.V[static_cast<unsigned long long>(d) * kBatchLanes + lane];
             }
             if (use[q]) {
-              p.fn(vs(slot[t]), x[q], &ew[wib][i][j]);
-              vT const c = vs(slot[t]);
+              vT const c = edge_value(p.fn, slot[t], x[q], &ew[wib][i][j]);
               acc = c < acc ? c : acc;
             }
           }

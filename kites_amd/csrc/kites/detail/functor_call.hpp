@@ -9,6 +9,7 @@
 // from its signature: a plain reference does not bind to a volatile lvalue.
 //
 // The *_at forms work on LDS slots in place; edge_value returns the partial.
+// (The host's probe of a functor set calls them on locals.)
 #ifndef KITES_DETAIL_FUNCTOR_CALL_HPP_
 #define KITES_DETAIL_FUNCTOR_CALL_HPP_
 
@@ -26,7 +27,7 @@ __host__ __device__ __forceinline__ volatile T& as_volatile(T& x) {
 
 // nbrCompF(partial, srcV, edge); `slot`: an LDS slot of the calling lane.
 template <class FN, class vT, class eT>
-__device__ __forceinline__ vT edge_value(FN& fn, vT& slot, vT src, eT* edge) {
+__host__ __device__ __forceinline__ vT edge_value(FN& fn, vT& slot, vT src, eT* edge) {
   if constexpr (std::is_invocable<FN&, volatile vT&, vT, eT*>::value) {
     fn(as_volatile(slot), src, edge);
     return slot;
@@ -38,7 +39,7 @@ __device__ __forceinline__ vT edge_value(FN& fn, vT& slot, vT src, eT* edge) {
 }
 
 template <class FN, class vT, class eT>
-__device__ __forceinline__ void edge_value_at(FN& fn, vT& slot, vT src, eT* edge) {
+__host__ __device__ __forceinline__ void edge_value_at(FN& fn, vT& slot, vT src, eT* edge) {
   if constexpr (std::is_invocable<FN&, volatile vT&, vT, eT*>::value) {
     fn(as_volatile(slot), src, edge);
   } else {
@@ -50,7 +51,7 @@ __device__ __forceinline__ void edge_value_at(FN& fn, vT& slot, vT src, eT* edge
 
 // initF(local, global)
 template <class FI, class vT>
-__device__ __forceinline__ void init_at(FI& fi, vT& slot, vT global) {
+__host__ __device__ __forceinline__ void init_at(FI& fi, vT& slot, vT global) {
   vT g = global;
   if constexpr (std::is_invocable<FI&, volatile vT&, vT&>::value) {
     fi(as_volatile(slot), g);
@@ -63,7 +64,7 @@ __device__ __forceinline__ void init_at(FI& fi, vT& slot, vT global) {
 
 // redF(lhs, rhs)
 template <class FR, class vT>
-__device__ __forceinline__ void reduce_at(FR& fr, vT& lhs, vT& rhs) {
+__host__ __device__ __forceinline__ void reduce_at(FR& fr, vT& lhs, vT& rhs) {
   if constexpr (std::is_invocable<FR&, volatile vT&, volatile vT&>::value) {
     fr(as_volatile(lhs), as_volatile(rhs));
   } else {
@@ -75,7 +76,7 @@ __device__ __forceinline__ void reduce_at(FR& fr, vT& lhs, vT& rhs) {
 
 // updF(newV, oldV)
 template <class FU, class vT>
-__device__ __forceinline__ bool update_at(FU& fu, vT& slot, vT old) {
+__host__ __device__ __forceinline__ bool update_at(FU& fu, vT& slot, vT old) {
   if constexpr (std::is_invocable<FU&, volatile vT&, vT>::value) {
     return fu(as_volatile(slot), old);
   } else {
@@ -83,6 +84,33 @@ __device__ __forceinline__ bool update_at(FU& fu, vT& slot, vT old) {
     bool const u = fu(nv, old);
     slot = nv;
     return u;
+  }
+}
+
+// nv = redF(old, cand); returns updF(nv, old).  `work` and `slot`: LDS slots of
+// the lane, `slot` holding `cand`.
+template <class FR, class FU, class vT>
+__host__ __device__ __forceinline__ bool combine(FR& fr, FU& fu, vT old, vT cand, vT& work, vT& slot,
+                                        vT& nv) {
+  if constexpr (std::is_invocable<FR&, volatile vT&, volatile vT&>::value) {
+    as_volatile(work) = old;
+    fr(as_volatile(work), as_volatile(slot));
+    bool const u = update_at(fu, work, old);
+    nv = as_volatile(work);
+    return u;
+  } else {
+    vT l = old, r = cand;
+    fr(l, r);
+    if constexpr (std::is_invocable<FU&, volatile vT&, vT>::value) {
+      as_volatile(work) = l;
+      bool const u = fu(as_volatile(work), old);
+      nv = as_volatile(work);
+      return u;
+    } else {
+      bool const u = fu(l, old);
+      nv = l;
+      return u;
+    }
   }
 }
 

@@ -301,10 +301,7 @@ __global__ __launch_bounds__(kPersistBlock) void persist_kernel(P p) {
 #pragma unroll
         for (unsigned k = 0; k < kEPT; ++k) {
           cand[k] = vT{};
-          if (ok[k]) {
-            p.fn(vs(sm.slot[t]), sm.val[own[k]], p.oE + idx[k]);
-            cand[k] = sm.slot[t];
-          }
+          if (ok[k]) cand[k] = edge_value(p.fn, sm.slot[t], sm.val[own[k]], p.oE + idx[k]);
         }
         // One returning atomic min per edge (a filtering read first would
         // cost this one compute unit a second scattered access per edge);

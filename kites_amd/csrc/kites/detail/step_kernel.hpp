@@ -33,8 +33,9 @@
 // iteration statistics the schedulers read.
 //
 // User functors keep the reference signatures with volatile references
-// (README.md:16-23).  Each lane owns LDS slots that the functors operate on,
-// so no operand is forced into scratch memory.
+// (README.md:16-23): each lane owns LDS slots that they operate on, so no
+// operand is forced into scratch memory.  Functors with plain references work
+// on registers (functor_call.hpp).
 #ifndef KITES_DETAIL_STEP_KERNEL_HPP_
 #define KITES_DETAIL_STEP_KERNEL_HPP_
 
@@ -45,6 +46,7 @@
 #include <type_traits>
 
 #include "../common.hpp"
+#include "functor_call.hpp"
 #include "mlp_device.hpp"
 #include "ticket.hpp"
 #include "wave.hpp"
@@ -397,11 +399,6 @@ __device__ __forceinline__ void note_far(lane_acc& la, vT v) {
   la.vmin = x < la.vmin ? x : la.vmin;
 }
 
-template <class T>
-__device__ __forceinline__ volatile T& vs(T& x) {
-  return *reinterpret_cast<volatile T*>(&x);
-}
-
 // Keeps a loaded value alive without using it (forces the load).
 template <class T>
 __device__ __forceinline__ void keep_live(T const& x) {
@@ -722,46 +719,41 @@ __device__ __forceinline__ void block_flush(iter_ctx& c, step_smem<vT>& sm, grou
   }
 }
 
+// Relaxes V[v] with the partial `cand`; true if V[v] moved.  Delta variants
+// only.  `slot` and `work`: LDS slots of the lane (functors with volatile
+// references).  V only moves one way, so a candidate that does not improve on
+// a plain, possibly stale, read does not improve on the value either.
 template <bool MIN_FAST, class P, class vT>
-__device__ __forceinline__ bool relax(P& p, unsigned v, vT& cand, vT& work);
+__device__ __forceinline__ bool relax(P& p, unsigned v, vT cand, vT& slot, vT& work) {
+  if constexpr (MIN_FAST) {
+    if (!(cand < p.V[v])) return false;
+    vT const old = atomic_min_any(p.V + v, cand);
+    return cand < old;
+  } else {
+    vT old = p.V[v];
+    for (;;) {
+      vT nv{};
+      if (!combine(p.fr, p.fu, old, cand, work, slot, nv)) return false;
+      vT const prev = atomic_cas_global(p.V + v, old, nv);
+      if (prev == old) return true;
+      old = prev;
+    }
+  }
+}
 
-// Push-side relax of V[v] with the partial value in `cand`.  With native
+// Push-side relax of V[v] with the partial value `cand`.  With native
 // min the atomic does not return: the result is "v may have moved" (the
 // candidate beat a plain read of V[v]), which at worst enqueues v once
 // more than needed -- an extra, harmless relaxation next iteration -- and
 // saves the atomic's round trip.
 template <bool MIN_FAST, class P, class vT>
-__device__ __forceinline__ bool relax_push(P& p, unsigned v, vT& cand, vT& work) {
+__device__ __forceinline__ bool relax_push(P& p, unsigned v, vT cand, vT& slot, vT& work) {
   if constexpr (MIN_FAST) {
-    vT const cv = vs(cand);
-    if (!(cv < p.V[v])) return false;
-    atomic_min_any(p.V + v, cv);
+    if (!(cand < p.V[v])) return false;
+    atomic_min_any(p.V + v, cand);
     return true;
   } else {
-    return relax<false>(p, v, cand, work);
-  }
-}
-
-// Relaxes V[v] with the partial value in `cand` (LDS slot); true if V[v]
-// moved.  Delta variants only.
-template <bool MIN_FAST, class P, class vT>
-__device__ __forceinline__ bool relax(P& p, unsigned v, vT& cand, vT& work) {
-  if constexpr (MIN_FAST) {
-    vT const cv = vs(cand);
-    if (!(cv < p.V[v])) return false;
-    vT const old = atomic_min_any(p.V + v, cv);
-    return cv < old;
-  } else {
-    vT old = vs(p.V[v]);
-    for (;;) {
-      vs(work) = old;
-      p.fr(vs(work), vs(cand));
-      if (!p.fu(vs(work), old)) return false;
-      vT const nv = vs(work);
-      vT const prev = atomic_cas_global(p.V + v, old, nv);
-      if (prev == old) return true;
-      old = prev;
-    }
+    return relax<false>(p, v, cand, slot, work);
   }
 }
 
@@ -782,7 +774,7 @@ __device__ __forceinline__ bool seg_reduce(P& p, step_smem<vT>& sm, unsigned key
     if (same && hy) {
       if (has) {
         sm.rhs[t] = y;
-        p.fr(vs(sm.tmp[t]), vs(sm.rhs[t]));
+        reduce_at(p.fr, sm.tmp[t], sm.rhs[t]);
       } else {
         sm.tmp[t] = y;
         has = true;
@@ -888,8 +880,7 @@ __device__ void run_classic(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) 
     unsigned r0 = 0, deg = 0;
     if (active) {
       old = p.V[v];
-      vT g = old;
-      p.fi(vs(sm.acc[t]), g);
+      init_at(p.fi, sm.acc[t], old);
       r0 = p.R[v];
       deg = p.R[v + 1] - r0;
     }
@@ -909,7 +900,7 @@ __device__ void run_classic(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) 
         own = owner_search(excl, e);
         unsigned const idx = base[own] + (e - excl[own]);
         vT const sv = p.V[p.C[idx]];
-        p.fn(vs(sm.tmp[t]), sv, p.E + idx);
+        edge_value_at(p.fn, sm.tmp[t], sv, p.E + idx);
       }
       if constexpr (MIN_FAST) {
         if (valid) atomic_min_any(&sm.acc[(wib << 6) + own], sm.tmp[t]);
@@ -917,13 +908,13 @@ __device__ void run_classic(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) 
         bool const has = seg_reduce(p, sm, own, valid);
         unsigned const kprev = __shfl_up(own, 1, 64);
         bool const head = valid && has && (lane == 0 || kprev != own);
-        if (head) p.fr(vs(sm.acc[(wib << 6) + own]), vs(sm.tmp[t]));
+        if (head) reduce_at(p.fr, sm.acc[(wib << 6) + own], sm.tmp[t]);
       }
       wave_lds_sync();
     }
     bool upd = false;
     if (active) {
-      upd = p.fu(vs(sm.acc[t]), old);
+      upd = update_at(p.fu, sm.acc[t], old);
       if (upd) p.V[v] = sm.acc[t];
     }
     unsigned long long const umask = ballot64(upd);
@@ -1004,9 +995,9 @@ __device__ void run_push_thread(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& 
       if (i < deg) {
         unsigned const e = e0 + i;
         dst = p.oC[e];
-        p.fn(vs(sm.tmp[t]), val, p.oE + e);
-        if (relax_push<MIN_FAST>(p, dst, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
-          newly = claim_next(c, la, dst, vs(sm.tmp[t]), far);
+        vT const cand = edge_value(p.fn, sm.tmp[t], val, p.oE + e);
+        if (relax_push<MIN_FAST>(p, dst, cand, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
+          newly = claim_next(c, la, dst, cand, far);
       }
       append_queue(p, c, la, newly, dst);
       if (c.nf) far_append(c, far, dst);
@@ -1049,9 +1040,9 @@ __device__ void run_push_wave(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm
         unsigned const own = owner_search(excl, e);
         unsigned const idx = base[own] + (e - excl[own]);
         dst = p.oC[idx];
-        p.fn(vs(sm.tmp[t]), vals[own], p.oE + idx);
-        if (relax_push<MIN_FAST>(p, dst, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
-          newly = claim_next(c, la, dst, vs(sm.tmp[t]), far);
+        vT const cand = edge_value(p.fn, sm.tmp[t], vals[own], p.oE + idx);
+        if (relax_push<MIN_FAST>(p, dst, cand, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
+          newly = claim_next(c, la, dst, cand, far);
       }
       append_queue(p, c, la, newly, dst);
       if (c.nf) far_append(c, far, dst);
@@ -1079,9 +1070,9 @@ __device__ void run_push_block(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& s
       if (e < e1) {
         la.work += 1;
         dst = p.oC[e];
-        p.fn(vs(sm.tmp[t]), val, p.oE + e);
-        if (relax_push<MIN_FAST>(p, dst, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
-          newly = claim_next(c, la, dst, vs(sm.tmp[t]), far);
+        vT const cand = edge_value(p.fn, sm.tmp[t], val, p.oE + e);
+        if (relax_push<MIN_FAST>(p, dst, cand, sm.tmp[t], sm.rhs[t]) && has_out(p, dst))
+          newly = claim_next(c, la, dst, cand, far);
       }
       append_queue(p, c, la, newly, dst);
       if (c.nf) far_append(c, far, dst);
@@ -1146,8 +1137,7 @@ __device__ void run_pull_thread(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& 
             unsigned const s = p.C[e];
             if (test_bit(c.in_bm, s)) {
               la.gathers += 1;
-              p.fn(vs(sm.tmp[t]), p.V[s], p.E + e);
-              vT const cv = sm.tmp[t];
+              vT const cv = edge_value(p.fn, sm.tmp[t], p.V[s], p.E + e);
               acc = cv < acc ? cv : acc;
               ++e;
               break;
@@ -1160,8 +1150,7 @@ __device__ void run_pull_thread(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& 
             unsigned const s = p.C[e];
             if (test_bit(c.in_bm, s)) {
               la.gathers += 1;
-              p.fn(vs(sm.tmp[t]), p.V[s], p.E + e);
-              vT const cv = sm.tmp[t];
+              vT const cv = edge_value(p.fn, sm.tmp[t], p.V[s], p.E + e);
               acc = cv < acc ? cv : acc;
             }
           }
@@ -1170,17 +1159,16 @@ __device__ void run_pull_thread(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& 
         if (upd) p.V[v] = acc;
       } else {
         la.work += e1 - e0;
-        vT g = old;
-        p.fi(vs(sm.acc[t]), g);
+        init_at(p.fi, sm.acc[t], old);
         for (unsigned e = e0; e < e1; ++e) {
           unsigned const s = p.C[e];
           if (test_bit(c.in_bm, s)) {
             la.gathers += 1;
-            p.fn(vs(sm.tmp[t]), p.V[s], p.E + e);
-            p.fr(vs(sm.acc[t]), vs(sm.tmp[t]));
+            edge_value_at(p.fn, sm.tmp[t], p.V[s], p.E + e);
+            reduce_at(p.fr, sm.acc[t], sm.tmp[t]);
           }
         }
-        upd = p.fu(vs(sm.acc[t]), old);
+        upd = update_at(p.fu, sm.acc[t], old);
         if (upd) p.V[v] = sm.acc[t];
       }
     }
@@ -1202,8 +1190,7 @@ __device__ void run_pull_wave(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm
     unsigned r0 = 0, deg = 0;
     if (inr) {
       old = p.V[v];
-      vT g = old;
-      p.fi(vs(sm.acc[t]), g);
+      init_at(p.fi, sm.acc[t], old);
       r0 = p.R[v];
       deg = p.R[v + 1] - r0;
       la.active += 1;
@@ -1229,7 +1216,7 @@ __device__ void run_pull_wave(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm
         unsigned const s = p.C[idx];
         if (test_bit(c.in_bm, s)) {
           la.gathers += 1;
-          p.fn(vs(sm.tmp[t]), p.V[s], p.E + idx);
+          edge_value_at(p.fn, sm.tmp[t], p.V[s], p.E + idx);
           has = true;
         }
       }
@@ -1240,14 +1227,14 @@ __device__ void run_pull_wave(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm
           bool const h2 = seg_reduce(p, sm, own, has);
           unsigned const kprev = __shfl_up(own, 1, 64);
           bool const head = valid && h2 && (lane == 0 || kprev != own);
-          if (head) p.fr(vs(sm.acc[(wib << 6) + own]), vs(sm.tmp[t]));
+          if (head) reduce_at(p.fr, sm.acc[(wib << 6) + own], sm.tmp[t]);
         }
       }
       wave_lds_sync();
     }
     bool upd = false;
     if (inr) {
-      upd = p.fu(vs(sm.acc[t]), old);
+      upd = update_at(p.fu, sm.acc[t], old);
       if (upd) p.V[v] = sm.acc[t];
     }
     publish_word(p, c, la, upd, v, task);
@@ -1275,9 +1262,9 @@ __device__ void run_pull_block(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& s
         unsigned const s = p.C[e];
         if (test_bit(c.in_bm, s)) {
           la.gathers += 1;
-          p.fn(vs(sm.rhs[t]), p.V[s], p.E + e);
+          edge_value_at(p.fn, sm.rhs[t], p.V[s], p.E + e);
           if (has) {
-            p.fr(vs(sm.tmp[t]), vs(sm.rhs[t]));
+            reduce_at(p.fr, sm.tmp[t], sm.rhs[t]);
           } else {
             sm.tmp[t] = sm.rhs[t];
             has = true;
@@ -1292,7 +1279,7 @@ __device__ void run_pull_block(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& s
         if (lane < s && hy) {
           if (has) {
             sm.rhs[t] = y;
-            p.fr(vs(sm.tmp[t]), vs(sm.rhs[t]));
+            reduce_at(p.fr, sm.tmp[t], sm.rhs[t]);
           } else {
             sm.tmp[t] = y;
             has = true;
@@ -1306,14 +1293,13 @@ __device__ void run_pull_block(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& s
       __syncthreads();
       if (t == 0) {
         vT const old = p.V[v];
-        vT g = old;
-        p.fi(vs(sm.acc[0]), g);
+        init_at(p.fi, sm.acc[0], old);
         for (int w = 0; w < kWaves; ++w)
           if (sm.whas[w]) {
             sm.rhs[0] = sm.wpart[w];
-            p.fr(vs(sm.acc[0]), vs(sm.rhs[0]));
+            reduce_at(p.fr, sm.acc[0], sm.rhs[0]);
           }
-        if (p.fu(vs(sm.acc[0]), old)) {
+        if (update_at(p.fu, sm.acc[0], old)) {
           p.V[v] = sm.acc[0];
           sm.ubits |= 1ull << j;
         }
@@ -1509,8 +1495,7 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
 #pragma unroll
             for (unsigned i = 0; i < kIPL; ++i) {
               if (valid[i]) {
-                p.fn(vs(sm.tmp[t]), wval[j[i]], p.oE + idx[i]);
-                cand[i] = sm.tmp[t];
+                cand[i] = edge_value(p.fn, sm.tmp[t], wval[j[i]], p.oE + idx[i]);
               }
             }
             // Non-returning atomics: a candidate that beats the plain read
@@ -1535,8 +1520,8 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
             for (unsigned i = 0; i < kIPL; ++i) {
               newly[i] = false;
               if (valid[i]) {
-                p.fn(vs(sm.tmp[t]), wval[j[i]], p.oE + idx[i]);
-                if (relax<false>(p, dst[i], sm.tmp[t], sm.rhs[t]) && has_out(p, dst[i]))
+                vT const cand = edge_value(p.fn, sm.tmp[t], wval[j[i]], p.oE + idx[i]);
+                if (relax<false>(p, dst[i], cand, sm.tmp[t], sm.rhs[t]) && has_out(p, dst[i]))
                   newly[i] = set_bit_once(c.out_bm, dst[i]);
               }
             }
@@ -1606,8 +1591,7 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
               }
               if (hit[i]) {
                 la.gathers += 1;
-                p.fn(vs(sm.tmp[t]), sv[i], Ep + e[i]);
-                vT const cv = sm.tmp[t];
+                vT const cv = edge_value(p.fn, sm.tmp[t], sv[i], Ep + e[i]);
                 acc = (has && acc < cv) ? acc : cv;
                 has = true;
               }
@@ -1621,7 +1605,7 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
             for (unsigned i = 0; i < kIPL; ++i) {
               if (hit[i]) {
                 la.gathers += 1;
-                p.fn(vs(sm.tmp[t]), sv[i], Ep + e[i]);
+                edge_value_at(p.fn, sm.tmp[t], sv[i], Ep + e[i]);
               }
               if (ballot64(hit[i])) {
                 unsigned const key = valid[i] ? j[i] : 64 + lane;
@@ -1630,7 +1614,7 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
                 bool const head = valid[i] && h2 && (lane == 0 || kprev != key);
                 if (head) {
                   if (whas[j[i]]) {
-                    p.fr(vs(wslot[j[i]]), vs(sm.tmp[t]));
+                    reduce_at(p.fr, wslot[j[i]], sm.tmp[t]);
                   } else {
                     wslot[j[i]] = sm.tmp[t];
                     whas[j[i]] = 1;
@@ -1653,8 +1637,9 @@ __device__ void run_lb(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
             vT const pv = wslot[lane];
             moved = pv < wval[lane] && pv < atomic_min_any(p.V + vert, pv);
           } else {
-            sm.tmp[t] = wslot[lane];
-            moved = relax<false>(p, vert, sm.tmp[t], sm.rhs[t]);
+            vT const cand = wslot[lane];
+            sm.tmp[t] = cand;
+            moved = relax<false>(p, vert, cand, sm.tmp[t], sm.rhs[t]);
           }
           if (moved && wbase[lane] != 0) {
             unsigned long long const bit = 1ull << (vert & 63);

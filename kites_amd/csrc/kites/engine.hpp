@@ -39,6 +39,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "detail/functor_call.hpp"
 #include "detail/ordered_kernel.hpp"
 #include "detail/persist_kernel.hpp"
 #include "detail/step_kernel.hpp"
@@ -175,26 +176,25 @@ probe_result probe_functors(FI fi, FN, FR fr, FU fu) {
     while (k < s.size()) s[k++] = static_cast<vT>(rng());
     bool init_id = true, is_min = true, upd_lt = true, semi = true, upd_moved = true;
     auto red = [&](vT a, vT b) {
-      volatile vT l = a, rr = b;
-      fr(l, rr);
-      return static_cast<vT>(l);
+      vT l = a, rr = b;
+      reduce_at(fr, l, rr);
+      return l;
     };
     for (vT a : s) {
-      volatile vT loc{};
-      vT g = a;
-      fi(loc, g);
-      if (static_cast<vT>(loc) != a) init_id = false;
+      vT loc{};
+      init_at(fi, loc, a);
+      if (loc != a) init_id = false;
       if (red(a, a) != a) semi = false;
       for (vT b : s) {
         vT const ab = red(a, b);
         if (ab != std::min(a, b)) is_min = false;
         if (ab != red(b, a)) semi = false;
-        volatile vT nv = a;
-        bool const u = fu(nv, b);
+        vT nv = a;
+        bool const u = update_at(fu, nv, b);
         if (u != (a < b)) upd_lt = false;
         vT const rb = red(b, a);
-        volatile vT nv2 = rb;
-        if (fu(nv2, b) != (rb != b)) upd_moved = false;
+        vT nv2 = rb;
+        if (update_at(fu, nv2, b) != (rb != b)) upd_moved = false;
       }
     }
     for (std::size_t i = 0; i + 2 < s.size(); i += 3)

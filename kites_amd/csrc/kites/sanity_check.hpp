@@ -29,14 +29,15 @@ bool sanity_check(graph_csr<vT, eT, vIdxT>& h, graph_csr_device<vT, eT, vIdxT>& 
     any = false;
     for (std::size_t v = 0; v < n; ++v) {
       vT pre = h.V[v];
-      volatile vT inHand;
-      funcInit(inHand, pre);
+      vT inHand{};
+      detail::init_at(funcInit, inHand, pre);
       for (vIdxT e = h.R[v]; e < h.R[v + 1]; ++e) {
-        volatile vT tmp;
-        funcCompNbr(tmp, h.V.at(h.C.at(e)), h.E.get_ptr() + e);
-        funcRed(inHand, tmp);
+        vT tmp{};
+        detail::edge_value_at(funcCompNbr, tmp, static_cast<vT>(h.V.at(h.C.at(e))),
+                              h.E.get_ptr() + e);
+        detail::reduce_at(funcRed, inHand, tmp);
       }
-      if (funcUpd(inHand, pre)) {
+      if (detail::update_at(funcUpd, inHand, pre)) {
         h.V[v] = inHand;
         any = true;
       }
