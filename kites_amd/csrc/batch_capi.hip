@@ -130,14 +130,8 @@ int kites_batch_values(kites_graph* g, uint32_t* out) {
   need(g != nullptr && out != nullptr, "null argument");
   need(g->rows.size() >= static_cast<std::size_t>(g->n) * 64, "no multi-source run yet");
   g->dev->setAsActive();
-  if (g->batch_k == 64)   // whole rows: one contiguous copy
-    KITES_HIP_CHECK(hipMemcpy(out, g->rows.get_ptr(),
-                              static_cast<std::size_t>(g->n) * 64 * sizeof(unsigned),
-                              hipMemcpyDeviceToHost));
-  else if (g->batch_k)
-    KITES_HIP_CHECK(hipMemcpy2D(out, g->batch_k * sizeof(unsigned), g->rows.get_ptr(),
-                                64 * sizeof(unsigned), g->batch_k * sizeof(unsigned), g->n,
-                                hipMemcpyDeviceToHost));
+  kites_capi::copy_columns(out, g->rows.get_ptr(), g->n, 64u, g->batch_k, g->dev->getDevIdx(),
+                           g->dev->getSsEven().get());
   KITES_API_END
 }
 
@@ -271,14 +265,8 @@ int kites_bfs256_levels(kites_graph* g, uint32_t* out) {
   need(g != nullptr && out != nullptr, "null argument");
   need(g->levels.size() >= static_cast<std::size_t>(g->n) * 256, "no bit-parallel BFS run yet");
   g->dev->setAsActive();
-  if (g->bfs_k == 256)   // whole rows: one contiguous copy
-    KITES_HIP_CHECK(hipMemcpy(out, g->levels.get_ptr(),
-                              static_cast<std::size_t>(g->n) * 256 * sizeof(unsigned),
-                              hipMemcpyDeviceToHost));
-  else if (g->bfs_k)
-    KITES_HIP_CHECK(hipMemcpy2D(out, g->bfs_k * sizeof(unsigned), g->levels.get_ptr(),
-                                256 * sizeof(unsigned), g->bfs_k * sizeof(unsigned), g->n,
-                                hipMemcpyDeviceToHost));
+  kites_capi::copy_columns(out, g->levels.get_ptr(), g->n, 256u, g->bfs_k, g->dev->getDevIdx(),
+                           g->dev->getSsEven().get());
   KITES_API_END
 }
 

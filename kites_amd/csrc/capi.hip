@@ -492,8 +492,8 @@ int kites_graph_values(kites_graph* g, uint32_t* out) {
   KITES_API_BEGIN
   need(g != nullptr && out != nullptr, "null argument");
   g->dev->setAsActive();
-  KITES_HIP_CHECK(hipMemcpy(out, g->g->V.get_ptr(), g->n * sizeof(unsigned),
-                            hipMemcpyDeviceToHost));
+  kites_capi::copy_columns(out, g->g->V.get_ptr(), g->n, 1u, 1u, g->dev->getDevIdx(),
+                           g->dev->getSsEven().get());
   KITES_API_END
 }
 

@@ -13,6 +13,7 @@
 
 #include "../../include/kites_amd.h"
 #include "hgraph.hpp"
+#include "host_copy.hpp"
 #include "kites/kites.hpp"
 
 struct kites_hgraph {
@@ -20,6 +21,7 @@ struct kites_hgraph {
 };
 
 struct kites_graph {
+  kites_capi::copy_user copies;
   std::unique_ptr<kites::gpu> dev;
   std::unique_ptr<kites::graph_csr_device<unsigned, unsigned>> g;
   uint32_t n = 0;

@@ -98,7 +98,8 @@ int kites_pagerank_f32(kites_graph* g, float damping, float tol, uint32_t max_it
   o.report = &rep;
   kites::detail::run_ordered(f, dev, s, g->pr_ws, initF, nbrF, redF, updF, o);
   if (out && n)
-    KITES_HIP_CHECK(hipMemcpy(out, V, n * sizeof(float), hipMemcpyDeviceToHost));
+    kites_capi::copy_columns(reinterpret_cast<unsigned*>(out), reinterpret_cast<const unsigned*>(V),
+                             n, 1u, 1u, did, s.get());
   if (info) {
     info->iterations = rep.iterations;
     info->ms = static_cast<float>(rep.ms);
