@@ -43,22 +43,50 @@ __global__ void mark_out_kernel(const unsigned* oR, const unsigned* oC, unsigned
   }
 }
 
+// Unit start of a source list: one thread per source.
 __global__ void seed_values_kernel(unsigned* V, const unsigned* list, unsigned count,
-                                   unsigned value, unsigned long long* bm, const unsigned* oR,
-                                   const unsigned* oC) {
-  // one workgroup per source: its value, then its out-neighbours' frontier bits
+                                   unsigned value) {
+  unsigned const i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) V[list[i]] = value;
+}
+
+// The out-neighbours' frontier bits of a source list, one workgroup per source.
+__global__ void mark_list_kernel(const unsigned* list, unsigned count, unsigned long long* bm,
+                                 const unsigned* oR, const unsigned* oC) {
   unsigned const i = blockIdx.x;
   if (i >= count) return;
   unsigned const s = list[i];
-  if (threadIdx.x == 0) V[s] = value;
   for (unsigned e = oR[s] + threadIdx.x; e < oR[s + 1]; e += blockDim.x) {
     unsigned const v = oC[e];
     atomicOr(bm + (v >> 6), 1ull << (v & 63));
   }
 }
 
+unsigned fill_grid(unsigned n) { return std::min(1024u, std::max(1u, (n + 255u) / 256u)); }
 
 }  // namespace
+
+namespace kites_capi {
+
+// The reference protocol's frontier of a start recorded by kites_graph_init or
+// kites_graph_init_sources: the sources' out-neighbours (every vertex for
+// min-label CC is marked with the values).  Only the reference algorithm reads
+// it; delta schedules start from the recorded sources themselves.
+void mark_start(kites_graph* g) {
+  auto& dg = *g->g;
+  g->dev->setAsActive();
+  hipStream_t s = g->dev->getSsEven().get();
+  if (g->seed == kites::options::seeding::source)
+    hipLaunchKernelGGL(mark_out_kernel, dim3(64), dim3(256), 0, s, dg.oR.get_ptr(),
+                       dg.oC.get_ptr(), g->seed_source, dg.vBitmapEven.get_ptr());
+  else if (g->seed == kites::options::seeding::list && g->seed_count)
+    hipLaunchKernelGGL(mark_list_kernel, dim3(g->seed_count), dim3(256), 0, s,
+                       g->seed_list.get_ptr(), g->seed_count, dg.vBitmapEven.get_ptr(),
+                       dg.oR.get_ptr(), dg.oC.get_ptr());
+  KITES_HIP_CHECK(hipPeekAtLastError());
+}
+
+}  // namespace kites_capi
 
 extern "C" {
 
@@ -397,10 +425,10 @@ int kites_graph_init(kites_graph* g, int32_t algo, uint32_t source) {
   g->dev->setAsActive();
   hipStream_t s = g->dev->getSsEven().get();
   unsigned const nwords = static_cast<unsigned>(dg.vBitmapEven.size());
-  // The frontier written here is the reference protocol's (used by classic
-  // runs); delta runs start from the equivalent seed instead.
+  // Values and a cleared frontier (all set for CC).  Delta runs start from the
+  // recorded seed; a classic run marks its out-neighbours first (mark_start).
   if (algo == KITES_ALGO_CC) {
-    hipLaunchKernelGGL(fill_values_kernel, dim3(1024), dim3(256), 0, s, dg.V.get_ptr(), g->n, 0u,
+    hipLaunchKernelGGL(fill_values_kernel, dim3(fill_grid(g->n)), dim3(256), 0, s, dg.V.get_ptr(), g->n, 0u,
                        0u, 0u, 1, dg.vBitmapEven.get_ptr(), nwords, 1);
     g->seed = kites::options::seeding::all;
     g->unit_start = false;
@@ -414,11 +442,9 @@ int kites_graph_init(kites_graph* g, int32_t algo, uint32_t source) {
     // example's INF = 2^30 - 1 (sssp_basic_single_device.cu:20-21), which
     // cannot wrap; the other sets start from 0xFFFFFFFF.
     unsigned const fill = widest ? 0u : (algo == KITES_ALGO_SSSP_WRAP ? 1073741823u : kInf);
-    hipLaunchKernelGGL(fill_values_kernel, dim3(1024), dim3(256), 0, s, dg.V.get_ptr(), g->n,
+    hipLaunchKernelGGL(fill_values_kernel, dim3(fill_grid(g->n)), dim3(256), 0, s, dg.V.get_ptr(), g->n,
                        fill, source, widest ? kInf : 0u, 0,
                        dg.vBitmapEven.get_ptr(), nwords, 0);
-    hipLaunchKernelGGL(mark_out_kernel, dim3(64), dim3(256), 0, s, dg.oR.get_ptr(),
-                       dg.oC.get_ptr(), source, dg.vBitmapEven.get_ptr());
     g->seed = kites::options::seeding::source;
     g->seed_source = source;
     g->unit_start = fill == kInf && !widest;
@@ -450,13 +476,12 @@ int kites_graph_init_sources(kites_graph* g, int32_t algo, const uint32_t* sourc
     KITES_HIP_CHECK(hipMemcpyAsync(g->seed_list.get_ptr(), list.data(), list.size() * 4,
                                    hipMemcpyHostToDevice, s));
   // values = fill everywhere (no source: the fill kernel's source index is n)
-  hipLaunchKernelGGL(fill_values_kernel, dim3(1024), dim3(256), 0, s, dg.V.get_ptr(), g->n, fill,
+  hipLaunchKernelGGL(fill_values_kernel, dim3(fill_grid(g->n)), dim3(256), 0, s, dg.V.get_ptr(), g->n, fill,
                      g->n, 0u, 0, dg.vBitmapEven.get_ptr(), nwords, 0);
   if (!list.empty())
-    hipLaunchKernelGGL(seed_values_kernel, dim3(static_cast<unsigned>(list.size())), dim3(256), 0,
-                       s, dg.V.get_ptr(), g->seed_list.get_ptr(),
-                       static_cast<unsigned>(list.size()), 0u, dg.vBitmapEven.get_ptr(),
-                       dg.oR.get_ptr(), dg.oC.get_ptr());
+    hipLaunchKernelGGL(seed_values_kernel, dim3((static_cast<unsigned>(list.size()) + 255) / 256),
+                       dim3(256), 0, s, dg.V.get_ptr(), g->seed_list.get_ptr(),
+                       static_cast<unsigned>(list.size()), 0u);
   KITES_HIP_CHECK(hipPeekAtLastError());
   g->seed = kites::options::seeding::list;
   g->seed_count = static_cast<uint32_t>(list.size());
@@ -471,6 +496,7 @@ int kites_graph_run(kites_graph* g, int32_t algo, const kites_run_opts* o, kites
   kites::options opt = to_options(g, o);
   opt.report = &rep;
   settle_bfs(g, algo, opt);
+  if (opt.sched == kites::schedule::classic) kites_capi::mark_start(g);
   // The recorded start is consumed by this run, as the frontier is.
   g->seed = kites::options::seeding::none;
   g->unit_start = false;

@@ -69,6 +69,8 @@ inline int fail(std::exception const& e) {
   return KITES_ERR_OTHER;
 }
 
+void mark_start(kites_graph* g);   // capi.hip
+
 inline void need(bool c, const char* what) {
   if (!c) throw std::invalid_argument(what);
 }

@@ -10,9 +10,12 @@
 // on, so PCIe (57 GB/s), the page faults and the copies overlap.  Results of up
 // to kCopySmall bytes take one hipMemcpyAsync and one copy (12 us for 28 KB).
 //
-// The pinned buffers are kept between calls: at most kKeepRings in the
-// process, given back when the last graph handle is destroyed.  A buffer serves
-// one call at a time (concurrent calls take or make their own).
+// The pinned buffers (2 MB, or 16 MB for results above kCopyMiddle bytes) are
+// kept between calls: at most kKeepRings of each size in the process, all but
+// one small one given back when the last graph handle is destroyed (a program
+// that builds, solves and drops one graph after the other would pay 1.5 ms for
+// a large one each time).  A buffer serves one call at a time (concurrent calls
+// take or make their own).
 #ifndef KITES_AMD_HOST_COPY_HPP_
 #define KITES_AMD_HOST_COPY_HPP_
 
@@ -37,9 +40,10 @@ namespace kites_capi {
 constexpr unsigned kCopyThreads = 8;
 constexpr std::size_t kCopyBlock = std::size_t(1) << 14;    // bytes per flag
 constexpr std::size_t kCopyChunk = std::size_t(1) << 18;    // bytes a thread moves at a time
-constexpr std::size_t kCopyHalf = std::size_t(1) << 23;     // bytes of one launch
-constexpr std::size_t kCopySmall = std::size_t(1) << 20;
-constexpr unsigned kCopyBlocks = static_cast<unsigned>(kCopyHalf / kCopyBlock);
+constexpr std::size_t kCopyHalves[2] = {std::size_t(1) << 20, std::size_t(1) << 23};  // bytes of
+                                                            // one launch, small and large ring
+constexpr std::size_t kCopySmall = kCopyHalves[0];          // one hipMemcpyAsync up to here
+constexpr std::size_t kCopyMiddle = std::size_t(1) << 22;   // the small ring up to here
 // Workgroups of a launch: 64 blocks in flight keep PCIe busy, and blocks still
 // finish in order a megabyte at a time.
 constexpr unsigned kCopyGrid = 32;
@@ -49,22 +53,23 @@ constexpr std::size_t kKeepRings = 2;
 // of the launch that last filled the block).
 struct copy_ring {
   int device = -1;
+  std::size_t bytes;           // of a half
   unsigned char* mem = nullptr;
   unsigned launches = 0;       // numbers the launches of all calls it served
-  explicit copy_ring(int d) : device(d) {
-    KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&mem),
-                                  2 * (kCopyHalf + kCopyBlocks * sizeof(unsigned)),
+  copy_ring(int d, std::size_t half_bytes) : device(d), bytes(half_bytes) {
+    std::size_t const marks = 2 * (bytes / kCopyBlock) * sizeof(unsigned);
+    KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&mem), 2 * bytes + marks,
                                   hipHostMallocPortable | hipHostMallocCoherent));
-    std::memset(flags(0), 0, 2 * kCopyBlocks * sizeof(unsigned));
+    std::memset(mem + 2 * bytes, 0, marks);
   }
   copy_ring(copy_ring const&) = delete;
   copy_ring& operator=(copy_ring const&) = delete;
   ~copy_ring() {
     if (mem) (void)hipHostFree(mem);
   }
-  unsigned char* half(std::size_t launch) const { return mem + (launch & 1) * kCopyHalf; }
+  unsigned char* half(std::size_t launch) const { return mem + (launch & 1) * bytes; }
   unsigned* flags(std::size_t launch) const {
-    return reinterpret_cast<unsigned*>(mem + 2 * kCopyHalf) + (launch & 1) * kCopyBlocks;
+    return reinterpret_cast<unsigned*>(mem + 2 * bytes) + (launch & 1) * (bytes / kCopyBlock);
   }
 };
 
@@ -77,25 +82,27 @@ struct copy_pool {
     static copy_pool* const p = new copy_pool();
     return *p;
   }
-  std::unique_ptr<copy_ring> take(int device) {
+  std::unique_ptr<copy_ring> take(int device, std::size_t half) {
     {
       std::lock_guard<std::mutex> l(mu);
-      for (auto& r : idle)
-        if (r->device == device) {
-          std::unique_ptr<copy_ring> got = std::move(r);
-          idle.erase(idle.begin() + (&r - idle.data()));
+      for (std::size_t i = 0; i < idle.size(); ++i)
+        if (idle[i]->device == device && idle[i]->bytes == half) {
+          std::unique_ptr<copy_ring> got = std::move(idle[i]);
+          idle.erase(idle.begin() + static_cast<std::ptrdiff_t>(i));
           return got;
         }
     }
-    return std::unique_ptr<copy_ring>(new copy_ring(device));
+    return std::unique_ptr<copy_ring>(new copy_ring(device, half));
   }
   void give(std::unique_ptr<copy_ring> r) {
     std::lock_guard<std::mutex> l(mu);
-    if (handles && idle.size() < kKeepRings) idle.push_back(std::move(r));
+    std::size_t same = 0;
+    for (auto const& x : idle) same += x->bytes == r->bytes;
+    if (same < kKeepRings) idle.push_back(std::move(r));
   }
 };
 
-// Held by every graph handle: the last one to go gives the slots back.
+// Held by every graph handle: with the last one the pinned memory goes back.
 struct copy_user {
   copy_user() {
     auto& p = copy_pool::get();
@@ -108,7 +115,10 @@ struct copy_user {
     auto& p = copy_pool::get();
     std::vector<std::unique_ptr<copy_ring>> gone;
     std::lock_guard<std::mutex> l(p.mu);
-    if (--p.handles == 0) gone.swap(p.idle);
+    if (--p.handles) return;
+    gone.swap(p.idle);
+    for (auto& r : gone)
+      if (p.idle.empty() && r->bytes == kCopyHalves[0]) p.idle.push_back(std::move(r));
   }
 };
 
@@ -174,8 +184,9 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
   std::size_t const bytes = n * K * sizeof(unsigned);
   if (!bytes) return;
   auto& pool = copy_pool::get();
-  std::unique_ptr<copy_ring> ring = pool.take(device);
   KITES_HIP_CHECK(hipSetDevice(device));
+  std::size_t const half = kCopyHalves[bytes > kCopyMiddle];
+  std::unique_ptr<copy_ring> ring = pool.take(device, half);
   if (bytes <= kCopySmall && K == stride) {
     hipError_t const e = hipMemcpyAsync(ring->half(0), rows, bytes, hipMemcpyDeviceToHost, s);
     KITES_HIP_CHECK(hipStreamSynchronize(s));
@@ -184,13 +195,13 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
     pool.give(std::move(ring));
     return;
   }
-  std::size_t const launches = (bytes + kCopyHalf - 1) / kCopyHalf;
+  std::size_t const launches = (bytes + half - 1) / half;
   std::size_t const chunks = (bytes + kCopyChunk - 1) / kCopyChunk;
-  constexpr std::size_t kPerHalf = kCopyHalf / kCopyChunk;
+  std::size_t const per_half = half / kCopyChunk;
   unsigned const base = ring->launches + 1;      // launch l is number base + l
   if (base + launches < base || base + launches > 0xfffffff0ull) {
     // (the numbers ran out: start over with cleared flags)
-    ring.reset(new copy_ring(device));
+    ring.reset(new copy_ring(device, half));
   }
   unsigned const number = ring->launches + 1;
   ring->launches += static_cast<unsigned>(launches);
@@ -198,7 +209,7 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
   std::atomic<int> error{0};
   std::vector<std::atomic<unsigned>> moved(launches);   // chunks of each launch moved on
   for (auto& m : moved) m.store(0);
-  auto chunks_of = [&](std::size_t l) { return std::min(kPerHalf, chunks - l * kPerHalf); };
+  auto chunks_of = [&](std::size_t l) { return std::min(per_half, chunks - l * per_half); };
   std::mutex issue_mu;
   // Queues, in order, every launch whose half is free: launch l reuses the
   // half of l - 2, so all chunks of that one have to have been moved on (the
@@ -207,7 +218,7 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
     std::lock_guard<std::mutex> lock(issue_mu);
     for (std::size_t l = issued.load();
          l < launches && (l < 2 || moved[l - 2].load() == chunks_of(l - 2)); ++l) {
-      std::size_t const at = l * kCopyHalf, count = std::min(kCopyHalf, bytes - at);
+      std::size_t const at = l * half, count = std::min(half, bytes - at);
       hipLaunchKernelGGL(copy_out_kernel, dim3(kCopyGrid), dim3(256), 0, s, rows, stride, K,
                          static_cast<unsigned long long>(at / sizeof(unsigned)),
                          static_cast<unsigned>(count / sizeof(unsigned)),
@@ -223,7 +234,7 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
     for (;;) {
       std::size_t const c = next.fetch_add(1);
       if (c >= chunks) return;
-      std::size_t const l = c / kPerHalf, at = c * kCopyChunk, in = at - l * kCopyHalf;
+      std::size_t const l = c / per_half, at = c * kCopyChunk, in = at - l * half;
       std::size_t const count = std::min(kCopyChunk, bytes - at);
       unsigned const* const flag = ring->flags(l) + in / kCopyBlock;
       for (std::size_t b = 0; b * kCopyBlock < count; ++b) {

@@ -451,9 +451,10 @@ __global__ __launch_bounds__(kPersistBlock) void persist_kernel(P p) {
       if (lane == 0) {
         p.ctl->next_variant = next;
         p.ctl->iter = iter + 1;
-        p.ctl->small_next = stop         ? 0u
-                            : split_next ? (fn_next <= kSmallWork ? 1u : 0u)
-                                         : grid_level(next, count, sdeg);
+        unsigned const level = stop         ? 0u
+                               : split_next ? (fn_next <= kSmallWork ? 1u : 0u)
+                                            : grid_level(next, count, sdeg);
+        p.ctl->small_next = level;
         p.ctl->q_count = count;
         p.ctl->q_edges = sdeg;
         if constexpr (FAR) {
@@ -476,6 +477,13 @@ __global__ __launch_bounds__(kPersistBlock) void persist_kernel(P p) {
         sm.go = (!stop && persist_fits<FAR, vT>(iter + 1, next, count, sdeg, fn_next, max_edges))
                     ? 1u
                     : 0u;
+        // (the iterations of the loop are part of one launch: the count of
+        // launches does not move, and the host sees the loop's end)
+        if (p.progress && !sm.go)
+          __hip_atomic_store(p.progress,
+                             progress_pack(iter + 1, p.ctl->launches, level, stop,
+                                           stop && (count != 0 || split_next)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
     __builtin_amdgcn_s_waitcnt(0);

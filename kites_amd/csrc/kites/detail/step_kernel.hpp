@@ -132,6 +132,9 @@ constexpr unsigned long long kSmallWork = 1ull << 18;
 // iteration, 128 take 10.5, 256 take 11.1 and 16 take 12.1.
 constexpr unsigned long long kTinyWork = 1ull << 16;
 
+// Iterations from which on a small frontier is taken to stay small.
+constexpr unsigned kGrowIters = 16;
+
 // A push iteration (thread, wave or edge-balanced) runs on
 // ceil(work / kWorkPerGroup) workgroups, work = queue entries + out-edges,
 // clamped to [one per compute unit, the whole grid].  Measured on R-MAT
@@ -168,6 +171,7 @@ struct step_ctl {
   unsigned overflow;
   unsigned seed_count;   // queue length the first iteration consumes (seeded runs)
   unsigned small_next;   // host hint for the next chunk's grid: 0 full, 1 small, 2 tiny
+  unsigned launches;     // launches that ran an iteration (the host's progress word)
   // The queue the next iteration consumes (written with `iter`, so that an
   // iteration reads its input from this one line): length and out-edges.
   unsigned q_count;
@@ -186,6 +190,19 @@ struct step_ctl {
   unsigned far_sel;
   ticket_board board;         // completion-ticket counters (not copied to the host)
 };
+
+// The run's state after an iteration, in one word of host memory that the
+// closing workgroup stores: the host follows the run without a copy in the
+// stream (a copy of the control line cost about 13 us per chunk of launches).
+__host__ __device__ constexpr unsigned long long progress_pack(unsigned iter, unsigned launches,
+                                                               unsigned level, bool done,
+                                                               bool overflow) {
+  return static_cast<unsigned long long>(iter) |
+         (static_cast<unsigned long long>(launches & 0xffffffu) << 32) |
+         (static_cast<unsigned long long>(level & 3u) << 56) |
+         (static_cast<unsigned long long>(done) << 58) |
+         (static_cast<unsigned long long>(overflow) << 59);
+}
 
 struct sched_params {
   unsigned mode;
@@ -267,6 +284,7 @@ struct step_core {
   unsigned* board;      // completion-ticket counters (kTicketWords)
   unsigned max_outdeg;  // largest out-degree of the graph (0: unknown)
   unsigned persist_edges;  // persist_kernel: largest queue out-edge total it takes (0: off)
+  unsigned long long* progress;  // pinned host word (progress_pack), or null
   // Source-split in-CSR for the edge-balanced pull (used when xsplit != 0):
   // the in-edges grouped by part of their source (kSplitParts parts, a
   // 32-vertex line of V belongs to one part), each part's edges ordered by
@@ -1876,15 +1894,25 @@ __device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<v
         p.ctl->thresh = t < far_vmin ? ~0ull : t;
       }
     }
-    p.ctl->small_next = stop         ? 0u
-                        : split_next ? (far_n <= kSmallWork ? 1u : 0u)
-                                     : grid_level(next, count, sdeg);
+    // (the first iterations keep the full grid: the host picks the grid of
+    // launches a few iterations ahead, and a frontier that is small now may be
+    // large by then -- R-MAT frontiers grow tenfold per iteration)
+    unsigned const level = stop || iter + 1 < kGrowIters ? 0u
+                           : split_next                  ? (far_n <= kSmallWork ? 1u : 0u)
+                                                         : grid_level(next, count, sdeg);
+    unsigned const launches = p.ctl->launches + 1;
+    bool const over = stop && (count != 0 || split_next);
+    p.ctl->small_next = level;
+    p.ctl->launches = launches;
     p.ctl->q_count = count;
     p.ctl->q_edges = sdeg;
     if (stop) {
       p.ctl->done = 1;
-      if (count != 0 || split_next) p.ctl->overflow = 1;
+      if (over) p.ctl->overflow = 1;
     }
+    if (p.progress)
+      __hip_atomic_store(p.progress, progress_pack(iter + 1, launches, level, stop, over),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -2045,145 +2073,149 @@ static __global__ void zero_words_kernel(unsigned* __restrict__ p, unsigned coun
     p[i] = 0u;
 }
 
-// Resets the control block, the statistics and all three bitmap slots of a
-// run.
-static __global__ void reset_kernel(step_stats* stats, unsigned nstats, unsigned long long* bm_ring,
-                             unsigned nwords, step_ctl* ctl,
-                             unsigned first_variant, unsigned max_iter, unsigned* update_flag,
-                             group_stats* gst, unsigned* board, unsigned long long delta,
-                             unsigned long long* far_bm) {
+// Start of a run, in one launch: clears the statistics, the three bitmap
+// slots, the far bitmap, the ticket board and the group slots, writes the
+// control block, and loads the start.  SEED_NONE: the frontier bitmap (`fw`
+// words) is moved into slot 0 and consumed.  Seeded starts of delta runs (the
+// first iteration propagates from a given updated set instead of recomputing
+// an initial frontier; the frontier bitmap is only cleared): SEED_SOURCE
+// {src}; SEED_ALL every vertex (queue = identity, offsets = oR); SEED_LIST is
+// completed by seed_list_kernel.  Picks the first variant with the run's
+// scheduler.  (Five small launches and copies before the first iteration cost
+// about 35 us on a graph of 100,000 edges.)
+enum seed_mode : unsigned { SEED_NONE = 0, SEED_SOURCE = 1, SEED_ALL = 2, SEED_LIST = 3 };
+
+template <class P>
+__global__ void start_kernel(P p, unsigned nstats, unsigned first_variant, unsigned max_iter,
+                             unsigned mode, unsigned src, unsigned long long* frontier,
+                             unsigned fw) {
   unsigned const tid = blockIdx.x * blockDim.x + threadIdx.x;
   unsigned const nt = gridDim.x * blockDim.x;
   if (tid < kTicketGroups) {
-    gst[tid] = group_stats{};
-    gst[tid].vmin = ~0ull;
+    p.gst[tid] = group_stats{};
+    p.gst[tid].vmin = ~0ull;
   }
-  clear_ticket_board(board, tid, nt);
-  unsigned long long* sw = reinterpret_cast<unsigned long long*>(stats);
+  clear_ticket_board(p.board, tid, nt);
+  unsigned long long* const sw = reinterpret_cast<unsigned long long*>(p.stats);
   unsigned const nsw = nstats * (sizeof(step_stats) / 8);
   for (unsigned i = tid; i < nsw; i += nt) sw[i] = 0ull;
-  for (unsigned i = tid; i < 3 * nwords; i += nt) bm_ring[i] = 0ull;
-  if (far_bm)
-    for (unsigned i = tid; i < nwords; i += nt) far_bm[i] = 0ull;
-  if (tid == 0) {
+  for (unsigned w = tid; w < p.nwords || w < fw; w += nt) {
+    if (w < p.nwords) {
+      unsigned const lo = w * 64u;
+      unsigned long long word = 0;
+      if (mode == SEED_NONE) {
+        word = w < fw ? frontier[w] : 0ull;
+      } else if (mode == SEED_SOURCE) {
+        word = w == (src >> 6) ? 1ull << (src & 63) : 0ull;
+      } else if (mode == SEED_ALL && lo < p.n) {
+        word = (p.n - lo >= 64) ? ~0ull : ((1ull << (p.n - lo)) - 1ull);
+      }
+      p.bm[w] = word;
+      p.bm[p.nwords + w] = 0ull;
+      p.bm[2ull * p.nwords + w] = 0ull;
+      if (p.fbm) p.fbm[w] = 0ull;
+    }
+    if (w < fw) frontier[w] = 0ull;
+  }
+  if (mode == SEED_ALL) {
+    for (unsigned i = tid; i < p.n; i += nt) p.q[i] = i;
+    for (unsigned i = tid; i <= p.n; i += nt) p.qe[i] = p.oR[i];
+  }
+  if (blockIdx.x != 0 || threadIdx.x >= 64) return;
+  unsigned count = 0, maxdeg = 0;
+  unsigned long long sdeg = 0;
+  if (mode == SEED_SOURCE) {
+    count = 1;
+    maxdeg = p.oR[src + 1] - p.oR[src];
+    sdeg = maxdeg;
+  } else if (mode == SEED_ALL) {
+    count = p.n;
+    sdeg = p.m;
+  }
+  if (threadIdx.x == 0) {
+    if (mode == SEED_SOURCE) {
+      p.q[0] = src;
+      p.qe[0] = 0;
+      p.qe[1] = maxdeg;
+    }
+    step_ctl* const ctl = p.ctl;
     ctl->iter = 0;
     ctl->done = 0;
     ctl->next_variant = first_variant;
     ctl->max_iter = max_iter;
     ctl->overflow = 0;
-    ctl->seed_count = 0;
+    ctl->seed_count = count;
     ctl->small_next = 0;
+    ctl->launches = 0;
     ctl->q_count = 0;
     ctl->q_edges = 0;
     ctl->cache_key = 0xffffffffu;
     ctl->cache_variant = 0;
-    ctl->thresh = delta ? delta : ~0ull;
+    ctl->thresh = p.sched.delta ? p.sched.delta : ~0ull;
     ctl->thresh_prev = 0;
     ctl->far_vmin = ~0ull;
     ctl->far_n = 0;
     ctl->far_next = 0;
     ctl->far_sel = 0;
-    if (update_flag) *update_flag = 0;
+    if (p.update_flag) *p.update_flag = 0;
+  }
+  if (mode == SEED_SOURCE || mode == SEED_ALL) {
+    learned_in li;
+    if (p.sched.mode == SCHED_LEARNED && p.sched.mlp) mlp_load_lane(p.sched.mlp, li.w);
+    unsigned const v = choose_variant(p, count, sdeg, maxdeg, 0, li);
+    if (threadIdx.x == 0) p.ctl->next_variant = v;
   }
 }
 
-// Seeded start of a delta run: the first iteration propagates from a given
-// updated set instead of recomputing an initial frontier.  SEED_SOURCE:
-// {source}; SEED_ALL: every vertex (queue = identity, offsets = oR);
-// SEED_LIST: `count` distinct vertices from `list` (one workgroup scans
-// their out-degrees into the queue offsets).  Runs after reset_kernel;
-// picks the first variant with the run's scheduler.
-enum seed_mode : unsigned { SEED_NONE = 0, SEED_SOURCE = 1, SEED_ALL = 2, SEED_LIST = 3 };
-
+// Completes a SEED_LIST start after start_kernel: `count` distinct vertices
+// from `list` (one workgroup scans their out-degrees into the queue offsets).
 template <class P>
-__global__ void seed_kernel(P p, unsigned mode, unsigned src, const unsigned* list,
-                            unsigned list_count) {
+__global__ void seed_list_kernel(P p, const unsigned* list, unsigned list_count) {
   __shared__ unsigned wtot[COMPILE_TIME_DETERMINED_BLOCK_SIZE / WAVE_SIZE];
   __shared__ unsigned long long s_sum;
   __shared__ unsigned s_max;
-  unsigned const tid = blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned const nt = gridDim.x * blockDim.x;
-  if (mode == SEED_ALL) {
-    for (unsigned i = tid; i < p.n; i += nt) p.q[i] = i;
-    for (unsigned i = tid; i <= p.n; i += nt) p.qe[i] = p.oR[i];
-    for (unsigned w = tid; w < p.nwords; w += nt) {
-      unsigned const lo = w * 64u;
-      unsigned long long word = 0;
-      if (lo < p.n) word = (p.n - lo >= 64) ? ~0ull : ((1ull << (p.n - lo)) - 1ull);
-      p.bm[w] = word;
-    }
+  // Block-wide exclusive scan of the out-degrees, 256 entries at a time.
+  unsigned const t = threadIdx.x, lane = lane_id(), wib = t >> 6;
+  if (t == 0) {
+    s_sum = 0;
+    s_max = 0;
   }
-  if (mode == SEED_LIST && blockIdx.x == 0) {
-    // Block-wide exclusive scan of the out-degrees, 256 entries at a time.
-    unsigned const t = threadIdx.x, lane = lane_id(), wib = t >> 6;
-    if (t == 0) {
-      s_sum = 0;
-      s_max = 0;
+  __syncthreads();
+  for (unsigned base = 0; base < list_count; base += blockDim.x) {
+    unsigned const i = base + t;
+    unsigned v = 0, d = 0;
+    if (i < list_count) {
+      v = list[i];
+      d = p.oR[v + 1] - p.oR[v];
+    }
+    unsigned const incl = wave_incl_scan(d);
+    if (lane == 63) wtot[wib] = incl;
+    __syncthreads();
+    unsigned before = 0, total = 0;
+    for (unsigned w = 0; w < blockDim.x / WAVE_SIZE; ++w) {
+      if (w < wib) before += wtot[w];
+      total += wtot[w];
+    }
+    unsigned const carry = static_cast<unsigned>(s_sum);
+    if (i < list_count) {
+      p.q[i] = v;
+      p.qe[i] = carry + before + incl - d;
+      atomicOr(p.bm + (v >> 6), 1ull << (v & 63));
+      atomicMax(&s_max, d);
     }
     __syncthreads();
-    for (unsigned base = 0; base < list_count; base += blockDim.x) {
-      unsigned const i = base + t;
-      unsigned v = 0, d = 0;
-      if (i < list_count) {
-        v = list[i];
-        d = p.oR[v + 1] - p.oR[v];
-      }
-      unsigned const incl = wave_incl_scan(d);
-      if (lane == 63) wtot[wib] = incl;
-      __syncthreads();
-      unsigned before = 0, total = 0;
-      for (unsigned w = 0; w < blockDim.x / WAVE_SIZE; ++w) {
-        if (w < wib) before += wtot[w];
-        total += wtot[w];
-      }
-      unsigned const carry = static_cast<unsigned>(s_sum);
-      if (i < list_count) {
-        p.q[i] = v;
-        p.qe[i] = carry + before + incl - d;
-        atomicOr(p.bm + (v >> 6), 1ull << (v & 63));
-        atomicMax(&s_max, d);
-      }
-      __syncthreads();
-      if (t == 0) s_sum += total;
-      __syncthreads();
-    }
-    if (t == 0) p.qe[list_count] = static_cast<unsigned>(s_sum);
+    if (t == 0) s_sum += total;
     __syncthreads();
   }
-  if (blockIdx.x == 0 && threadIdx.x < 64) {
-    unsigned count;
-    unsigned long long sdeg;
-    unsigned maxdeg = 0;
-    if (mode == SEED_ALL) {
-      count = p.n;
-      sdeg = p.m;
-    } else if (mode == SEED_LIST) {
-      count = list_count;
-      sdeg = s_sum;
-      maxdeg = s_max;
-    } else {
-      unsigned const d = p.oR[src + 1] - p.oR[src];
-      if (threadIdx.x == 0) {
-        p.q[0] = src;
-        p.qe[0] = 0;
-        p.qe[1] = d;
-        p.bm[src >> 6] |= 1ull << (src & 63);
-      }
-      count = 1;
-      sdeg = d;
-      maxdeg = d;
-    }
-    learned_in li;
-    if (p.sched.mode == SCHED_LEARNED && p.sched.mlp) {
-      li.cache_key = p.ctl->cache_key;
-      li.cache_variant = p.ctl->cache_variant;
-      mlp_load_lane(p.sched.mlp, li.w);
-    }
-    unsigned const v = choose_variant(p, count, sdeg, maxdeg, 0, li);
-    if (threadIdx.x == 0) {
-      p.ctl->seed_count = count;
-      p.ctl->next_variant = v;
-    }
+  if (t == 0) p.qe[list_count] = static_cast<unsigned>(s_sum);
+  __syncthreads();
+  if (t >= 64) return;
+  learned_in li;
+  if (p.sched.mode == SCHED_LEARNED && p.sched.mlp) mlp_load_lane(p.sched.mlp, li.w);
+  unsigned const v = choose_variant(p, list_count, s_sum, s_max, 0, li);
+  if (t == 0) {
+    p.ctl->seed_count = list_count;
+    p.ctl->next_variant = v;
   }
 }
 

@@ -239,6 +239,8 @@ struct run_state {
   step_ctl* ctl_host = nullptr;      // host memory the control header is copied into (two
                                      // slots when evc is set, else one)
   hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the copy into each slot (pipelining)
+  unsigned long long* progress = nullptr;  // pinned word the device reports to (null: copies of
+                                           // the control line)
   launch_cache* graphs = nullptr;    // null: iteration chunks are launched directly
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // null: the host clock times the run
 };
@@ -261,6 +263,7 @@ inline run_state state_of(workspace& ws) {
   st.ev1 = ws.ev1;
   st.evc[0] = ws.evc[0];
   st.evc[1] = ws.evc[1];
+  st.progress = ws.progress;
   return st;
 }
 
@@ -273,33 +276,68 @@ inline unsigned tiny_grid_of(gpu& dev, options const& o) {
                      : std::max(1u, static_cast<unsigned>(dev.numComputeUnits()) / 4u);
 }
 
-// Replays chunks of `chunk` launches until the run is done.  Every launch
-// of one chunk uses the same grid, picked from the state the last finished
-// chunk left (ctl.small_next): the full grid; one workgroup per compute
-// unit after a small push frontier (entries + out-edges <= kSmallWork);
-// a quarter of that after a tiny one (<= kTinyWork).  Small grids cut the
-// fixed cost of an iteration on long runs of small frontiers (high-diameter
-// graphs).  Within a launch, a push iteration does its work on as many
-// workgroups as its queue needs (at least prm.small_grid), and the rest
-// only count in.  With options::persist a tiny-grid chunk starts with
-// persist_kernel, which runs the iterations that fit one workgroup until
-// the frontier outgrows it; the chunk's step launches take the iterations
-// after that (or return at once when the run is done).
+// What the host knows of a run.
+struct run_progress {
+  unsigned iter, launches, level;
+  bool done, overflow;
+};
+
+inline run_progress read_progress(const unsigned long long* word) {
+  unsigned long long const w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+  return {static_cast<unsigned>(w), static_cast<unsigned>(w >> 32) & 0xffffffu,
+          static_cast<unsigned>(w >> 56) & 3u, ((w >> 58) & 1u) != 0, ((w >> 59) & 1u) != 0};
+}
+
+inline run_progress progress_of(step_ctl const& c) {
+  return {c.iter, c.launches & 0xffffffu, c.small_next, c.done != 0, c.overflow != 0};
+}
+
+// Launches queued ahead of the running one on the full and the small grid:
+// iterations there take 10 us and more, a launch costs the host about 4 us, so
+// single launches keep up, and a finished run has few that find nothing to do
+// (4.6 us each on the full grid; the end of a captured chunk costs 8 us).
+constexpr unsigned kAhead = 3;
+
+// Queues iterations until the run is done: single launches on the full and
+// the small grid, captured chunks of options::chunk launches on the tiny grid
+// and on small graphs.  The grid is picked from the run's state (grid_level): the
+// full grid; one workgroup per compute unit after a small push frontier
+// (entries + out-edges <= kSmallWork); a quarter of that after a tiny one
+// (<= kTinyWork).  Small grids cut the fixed cost of an iteration on long
+// runs of small frontiers (high-diameter graphs).  Within a launch, a push
+// iteration does its work on as many workgroups as its queue needs (at least
+// prm.small_grid), and the rest only count in.  With options::persist a
+// tiny-grid chunk starts with persist_kernel, which runs the iterations that
+// fit one workgroup until the frontier outgrows it; the chunk's step launches
+// take the iterations after that (or return at once when the run is done).
 //
-// The first chunk is waited for (short runs end in it).  After that, with
-// options::pipeline and the run state's copy events, the next chunk is
-// queued before the previous one's control line is read, so the host's
-// round trip overlaps device work; its grid comes from the chunk before,
-// and a chunk queued after the run is done only returns at once.
+// A graph whose vertices and edges together are at most kSmallWork never
+// leaves the small grid: all its chunks run there, from one captured
+// executable that starts with persist_kernel.
+//
+// The host follows the run through the progress word and queues more while
+// launches are left, so its round trip overlaps device work; launches
+// queued after the run is done only return at once.  Without the word
+// (caller-owned run states), or with options::pipeline off, the control line is
+// copied back after every chunk.
 template <bool DELTA, bool MIN_FAST, bool NF, class P>
 unsigned run_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options const& o,
                   run_state const& st) {
   auto kern = &step_kernel<DELTA, MIN_FAST, NF, P>;
   unsigned const chunk = std::max(1u, o.chunk);
+  bool const follow = prm.progress && o.pipeline;
+  bool const small_graph =
+      DELTA && o.adaptive_grid && !o.grid &&
+      static_cast<unsigned long long>(prm.n) + prm.m <= kSmallWork;
   unsigned g[3];
-  g[0] = grid;
   g[1] = std::min(grid, small_grid_of(dev, o));
   g[2] = std::min(g[1], tiny_grid_of(dev, o));
+  g[0] = grid;
+  if (o.adaptive_grid && !o.grid) {
+    unsigned long long const want =
+        (static_cast<unsigned long long>(prm.n) + prm.m + kWorkPerGroup - 1) / kWorkPerGroup;
+    if (want < grid) g[0] = std::max(g[1], static_cast<unsigned>(want));
+  }
   bool const levels = o.adaptive_grid && g[1] < grid;
   void (*pre)(P) = nullptr;
   if constexpr (DELTA && MIN_FAST) {
@@ -313,63 +351,77 @@ unsigned run_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options cons
   // the cache is older than the three executables this run uses.
   hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   bool const graphs = o.use_graph && st.graphs;
-  bool const pipe = o.pipeline && st.evc[0] && st.evc[1];
-  auto issue = [&](unsigned lv, unsigned slot) {
-    if (graphs && !exec[lv]) {
-      exec[lv] = st.graphs->chunk(kern, g[lv], COMPILE_TIME_DETERMINED_BLOCK_SIZE, chunk, prm,
-                                  s.get(), lv == 2 ? pre : nullptr, kPersistBlock);
-    }
-    if (exec[lv]) {
+  auto issue = [&](unsigned lv) {
+    bool const with_pre = pre && (lv == 2 || small_graph);
+    unsigned const count = follow && lv < 2 && !small_graph ? 1u : chunk;
+    if (graphs && count > 1 && !exec[lv])
+      exec[lv] = st.graphs->chunk(kern, g[lv], COMPILE_TIME_DETERMINED_BLOCK_SIZE, count, prm,
+                                  s.get(), with_pre ? pre : nullptr, kPersistBlock);
+    if (count > 1 && exec[lv]) {
       KITES_HIP_CHECK(hipGraphLaunch(exec[lv], s.get()));
     } else {
-      if (lv == 2 && pre)
-        hipLaunchKernelGGL(pre, dim3(1), dim3(kPersistBlock), 0, s.get(), prm);
-      for (unsigned k = 0; k < chunk; ++k)
+      if (with_pre) hipLaunchKernelGGL(pre, dim3(1), dim3(kPersistBlock), 0, s.get(), prm);
+      for (unsigned k = 0; k < count; ++k)
         hipLaunchKernelGGL(kern, dim3(g[lv]), dim3(COMPILE_TIME_DETERMINED_BLOCK_SIZE), 0,
                            s.get(), prm);
       KITES_HIP_CHECK(hipPeekAtLastError());
     }
-    KITES_HIP_CHECK(hipMemcpyAsync(st.ctl_host + slot, st.ctl, offsetof(step_ctl, board),
-                                   hipMemcpyDeviceToHost, s.get()));
-    if (pipe) KITES_HIP_CHECK(hipEventRecord(st.evc[slot], s.get()));
+    return count;
   };
-  auto level_of = [&](step_ctl const& c) { return levels ? std::min(c.small_next, 2u) : 0u; };
+  auto level_of = [&](run_progress const& c) {
+    return small_graph ? 1u : levels ? std::min(c.level, 2u) : 0u;
+  };
   unsigned long long const cap = static_cast<unsigned long long>(st.max_iter) + chunk;
-  unsigned long long launched = chunk;
-  issue(0, 0);
-  s.sync();
-  if (st.ctl_host[0].done) return static_cast<unsigned>(launched);
-  unsigned lv = level_of(st.ctl_host[0]);
-  if (!pipe) {
-    while (launched <= cap) {
-      issue(lv, 0);
-      launched += chunk;
+  unsigned long long launched = 0;
+  unsigned lv = small_graph ? 1u : 0u;
+  if (!follow) {
+    for (;;) {
+      launched += issue(lv);
+      KITES_HIP_CHECK(hipMemcpyAsync(st.ctl_host, st.ctl, offsetof(step_ctl, board),
+                                     hipMemcpyDeviceToHost, s.get()));
       s.sync();
-      if (st.ctl_host[0].done) break;
-      lv = level_of(st.ctl_host[0]);
+      run_progress const c = progress_of(*st.ctl_host);
+      if (c.done || launched > cap) break;
+      lv = level_of(c);
     }
     return static_cast<unsigned>(launched);
   }
-  // slot: the chunk whose control line is read next; last: the last queued
-  unsigned slot = 0, last = 0;
-  issue(lv, slot);
-  launched += chunk;
+  unsigned ahead = kAhead;
+  unsigned spins = 0;
+  auto since = std::chrono::steady_clock::now();
+  run_progress last{};
   for (;;) {
-    bool const more = launched <= cap;
-    if (more) {
-      last = slot ^ 1u;
-      issue(lv, last);
-      launched += chunk;
+    run_progress const c = read_progress(prm.progress);
+    if (c.done) break;
+    unsigned const left = static_cast<unsigned>(launched - c.launches) & 0xffffffu;
+    if (left <= ahead) {
+      if (launched > cap) break;
+      if (launched) lv = level_of(c);
+      unsigned const k = issue(lv);
+      launched += k;
+      ahead = k > 1 ? (small_graph ? std::min(kAhead, k / 2) : k / 2) : kAhead;
+      continue;
     }
-    KITES_HIP_CHECK(hipEventSynchronize(st.evc[slot]));
-    step_ctl const& c = st.ctl_host[slot];
-    if (c.done || !more) break;
-    lv = level_of(c);
-    slot ^= 1u;
+    if (c.iter != last.iter || c.launches != last.launches) {
+      last = c;
+      spins = 0;
+      since = std::chrono::steady_clock::now();
+    }
+    __builtin_ia32_pause();
+    // a stream that has failed reports nothing more
+    if (++spins % 65536 == 0 &&
+        std::chrono::steady_clock::now() - since > std::chrono::seconds(2)) {
+      hipError_t const e = hipStreamQuery(s.get());
+      if (e != hipErrorNotReady) {
+        KITES_HIP_CHECK(e);
+        if (!read_progress(prm.progress).done &&
+            read_progress(prm.progress).launches == c.launches)
+          throw std::runtime_error("kites::process: the queued iterations did not run");
+      }
+      since = std::chrono::steady_clock::now();
+    }
   }
   s.sync();
-  // the caller reads the final control line from the first slot
-  if (last != 0) st.ctl_host[0] = st.ctl_host[last];
   return static_cast<unsigned>(launched);
 }
 
@@ -784,6 +836,7 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   prm.sched.settled_below = o.settled_below;
   prm.sched.mlp = o.mlp_weights;
   prm.collect = (o.keep_stats || o.record) ? 1u : 0u;
+  prm.progress = o.record ? nullptr : st.progress;
   prm.gst = st.gst;
   prm.board = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(st.ctl) +
                                           offsetof(step_ctl, board));
@@ -806,35 +859,31 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
 
   auto const t0 = std::chrono::steady_clock::now();
   if (st.ev0) KITES_HIP_CHECK(hipEventRecord(st.ev0, s.get()));
-  // Reset the run state (all three bitmap slots included), then load the
-  // initial frontier (consumed, as the reference leaves both of its bitmaps
-  // empty after a run).
-  hipLaunchKernelGGL(reset_kernel, dim3(256), dim3(256), 0, s.get(), prm.stats, st.max_iter,
-                     prm.bm, st.nwords, prm.ctl,
-                     static_cast<unsigned>(sch == schedule::classic ? V_CLASSIC : V_INIT_LB),
-                     std::min(st.max_iter, std::max(2u, o.max_iterations)), prm.update_flag,
-                     prm.gst, prm.board, static_cast<unsigned long long>(o.delta), prm.fbm);
-  KITES_HIP_CHECK(hipPeekAtLastError());
+  // Clear the run state and load the start; the initial frontier is consumed
+  // (the reference leaves both of its bitmaps empty after a run).
+  unsigned const mode = o.seed == options::seeding::source ? SEED_SOURCE
+                        : o.seed == options::seeding::all  ? SEED_ALL
+                        : o.seed == options::seeding::list ? SEED_LIST
+                                                           : SEED_NONE;
+  if (prm.progress) __atomic_store_n(prm.progress, 0ull, __ATOMIC_RELEASE);
   std::size_t const fb = std::min<std::size_t>(grph.vBitmapEven.sizeInBytes(),
                                                st.nwords * sizeof(unsigned long long));
-  if (fb) {
-    KITES_HIP_CHECK(hipMemcpyAsync(prm.bm, grph.vBitmapEven.get_ptr(), fb,
-                                   hipMemcpyDeviceToDevice, s.get()));
-    KITES_HIP_CHECK(hipMemsetAsync(grph.vBitmapEven.get_ptr(), 0, grph.vBitmapEven.sizeInBytes(),
-                                   s.get()));
+  auto const start = &start_kernel<P>;
+  hipLaunchKernelGGL(start, dim3(mode == SEED_ALL ? 1024 : 512),
+                     dim3(COMPILE_TIME_DETERMINED_BLOCK_SIZE), 0, s.get(), kp, st.max_iter,
+                     static_cast<unsigned>(sch == schedule::classic ? V_CLASSIC : V_INIT_LB),
+                     std::min(st.max_iter, std::max(2u, o.max_iterations)), mode, o.seed_source,
+                     grph.vBitmapEven.get_ptr(), static_cast<unsigned>(fb / 8));
+  if (mode == SEED_LIST) {
+    auto const list = &seed_list_kernel<P>;
+    hipLaunchKernelGGL(list, dim3(1), dim3(COMPILE_TIME_DETERMINED_BLOCK_SIZE), 0, s.get(), kp,
+                       o.seed_list, o.seed_count);
   }
-
-  if (o.seed != options::seeding::none) {
-    unsigned const mode = o.seed == options::seeding::source ? SEED_SOURCE
-                          : o.seed == options::seeding::all  ? SEED_ALL
-                                                              : SEED_LIST;
-    if (fb)
-      KITES_HIP_CHECK(hipMemsetAsync(prm.bm, 0, st.nwords * sizeof(unsigned long long), s.get()));
-    hipLaunchKernelGGL(seed_kernel<P>, dim3(mode == SEED_ALL ? 1024 : 1),
-                       dim3(COMPILE_TIME_DETERMINED_BLOCK_SIZE), 0, s.get(), kp, mode,
-                       o.seed_source, o.seed_list, o.seed_count);
-    KITES_HIP_CHECK(hipPeekAtLastError());
-  }
+  KITES_HIP_CHECK(hipPeekAtLastError());
+  // (a bitmap longer than the run's slots: vertex groups finer than 64 ids)
+  if (grph.vBitmapEven.sizeInBytes() > fb)
+    KITES_HIP_CHECK(hipMemsetAsync(reinterpret_cast<char*>(grph.vBitmapEven.get_ptr()) + fb, 0,
+                                   grph.vBitmapEven.sizeInBytes() - fb, s.get()));
 
   unsigned grid = 0;
   bool const use_delta = (sch != schedule::classic);
@@ -888,7 +937,7 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
     KITES_HIP_CHECK(hipEventElapsedTime(&ms, st.ev0, st.ev1));
   else
     ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  step_ctl const ctl = *st.ctl_host;
+  run_progress const ctl = prm.progress ? read_progress(prm.progress) : progress_of(*st.ctl_host);
   if (!ctl.done || ctl.overflow)
     throw std::runtime_error("kites::process: iteration limit reached before convergence");
   if (o.verbose) {

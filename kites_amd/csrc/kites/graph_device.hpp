@@ -116,6 +116,7 @@ struct workspace {
   device_buffer<step_stats> stats;
   device_buffer<step_ctl> ctl;
   host_pinned_buffer<step_ctl> ctl_host;
+  unsigned long long* progress = nullptr; // pinned host word the closing workgroups store
   device_buffer<group_stats> gst;         // per-group partial statistics
   ordered_workspace ord;                   // ordered runs (allocated by the first one)
   launch_cache graphs;                     // captured iteration chunks
@@ -167,7 +168,9 @@ struct workspace {
       ctl.alloc(1, dev);
       ctl_host.alloc(2);
       gst.alloc(kTicketGroups, dev);
-      // (reset_kernel writes all of the control block that a run reads, on the
+      KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&progress), sizeof(unsigned long long),
+                                    hipHostMallocPortable | hipHostMallocCoherent));
+      // (start_kernel writes all of the control block that a run reads, on the
       // run's own stream; a null-stream memset here would not be ordered
       // before it, the stream being a non-blocking one)
       KITES_HIP_CHECK(hipEventCreate(&ev0));
@@ -182,7 +185,11 @@ struct workspace {
     if (fq.size() == 0) fq.alloc(2 * (n ? n : 1), dev);
     if (fbm.size() == 0) fbm.alloc(nwords, dev);
   }
+  workspace() = default;
+  workspace(workspace const&) = delete;
+  workspace& operator=(workspace const&) = delete;
   ~workspace() {
+    if (progress) (void)hipHostFree(progress);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     for (hipEvent_t e : evc)

@@ -12,7 +12,7 @@
 // current; host code only ever passes that address to the kernels, never
 // the array's name (which names a host-side stand-in).
 //
-// The array keeps the last call's contents; the engine's reset kernel
+// The array keeps the last call's contents; the engine's start kernel
 // clears everything a run reads before it is written.  Calls on one device
 // share the array, so they are serialized by a per-device mutex here:
 // calls from several host threads to one device wait for each other
@@ -94,6 +94,7 @@ int kites_sssp_u32_noalloc(kites_graph* g, uint32_t source, const kites_run_opts
   int rc = kites_graph_init(g, KITES_ALGO_SSSP, source);
   if (rc) return rc;
   kites::options opt = kites_capi::to_options(g, o);
+  if (opt.sched == kites::schedule::classic) kites_capi::mark_start(g);
   g->seed = kites::options::seeding::none;   // the recorded start is consumed
 
   kites::detail::run_state st;

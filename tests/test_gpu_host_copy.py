@@ -1,7 +1,7 @@
 """Results copied out of device memory (csrc/host_copy.hpp): sizes around the
 single copy's limit (1 MiB), a thread's chunk (256 KiB), a flagged block (16
-KiB) and a launch's half of the pinned memory (8 MiB), whole rows and the first
-K columns of wider ones; every value must arrive."""
+KiB) and a launch's half of the pinned memory (1 MiB, 8 MiB above 4 MiB), whole
+rows and the first K columns of wider ones; every value must arrive."""
 import numpy as np
 import pytest
 
@@ -17,7 +17,8 @@ def _edgeless(n):
 
 
 @pytest.mark.parametrize("n", [1, 3, 4095, 4097, (1 << 18) - 1, 1 << 18, (1 << 18) + 1,
-                               (1 << 18) + 4099, (1 << 20) + 3, (1 << 21) - 1, (1 << 21) + 1,
+                               (1 << 18) + 4099, (1 << 19) + 1, (1 << 20) - 1,
+                               (1 << 20) + 3, (1 << 21) - 1, (1 << 21) + 1,
                                (1 << 22) + 65539])
 def test_values(n):
     case(f"values n={n}")
