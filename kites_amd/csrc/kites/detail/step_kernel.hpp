@@ -128,9 +128,15 @@ static_assert(sizeof(step_stats) == 56, "step_stats layout");
 constexpr unsigned long long kSmallWork = 1ull << 18;
 // At most this much work (entries + out-edges) the next chunk runs on the
 // tiny grid (a quarter workgroup per compute unit): on 2048 x 2048 grid
-// BFS (about 10^4 work per iteration) 64 workgroups take 10.3 us per
-// iteration, 128 take 10.5, 256 take 11.1 and 16 take 12.1.
+// BFS (about 10^4 work per iteration, run_push_few) 16 workgroups take 9.2 us
+// per iteration, 32 take 8.1, 48 and 64 take 8.0, 96 take 8.5 and 128 take 8.6;
+// 64 with close_few take 7.4 (the edge-balanced push with the general close
+// took 9.4).
 constexpr unsigned long long kTinyWork = 1ull << 16;
+
+// Largest out-degree of the graphs whose tiny push iterations deal whole queue
+// entries to the waves (run_push_few).
+constexpr unsigned kFewDegree = 64;
 
 // Iterations from which on a small frontier is taken to stay small.
 constexpr unsigned kGrowIters = 16;
@@ -172,6 +178,7 @@ struct step_ctl {
   unsigned seed_count;   // queue length the first iteration consumes (seeded runs)
   unsigned small_next;   // host hint for the next chunk's grid: 0 full, 1 small, 2 tiny
   unsigned launches;     // launches that ran an iteration (the host's progress word)
+  unsigned max_outdeg;   // largest out-degree of the graph (0: unknown)
   // The queue the next iteration consumes (written with `iter`, so that an
   // iteration reads its input from this one line): length and out-edges.
   unsigned q_count;
@@ -188,8 +195,26 @@ struct step_ctl {
   unsigned far_n;
   unsigned far_next;
   unsigned far_sel;
+  // run_push_few's close on small grids: workgroups arrived, entries and
+  // out-edges appended, in one word (few_pack) on a line of its own.
+  alignas(128) unsigned long long few;
   ticket_board board;         // completion-ticket counters (not copied to the host)
 };
+
+// Workgroups (8 bits), entries (24) and out-edges (32) of a tiny iteration on a
+// graph of short out-lists: at most kTinyWork edges are expanded, each appends
+// at most one entry of at most kFewDegree out-edges.
+constexpr unsigned kFewGrid = 64;
+__host__ __device__ constexpr unsigned long long few_pack(unsigned groups, unsigned count,
+                                                          unsigned edges) {
+  return (static_cast<unsigned long long>(groups) << 56) |
+         (static_cast<unsigned long long>(count) << 32) | edges;
+}
+__host__ __device__ constexpr unsigned few_count(unsigned long long w) {
+  return static_cast<unsigned>(w >> 32) & 0xffffffu;
+}
+static_assert(kTinyWork < (1ull << 24) && kTinyWork * kFewDegree < (1ull << 32) && kFewGrid < 256,
+              "few_pack fields");
 
 // The run's state after an iteration, in one word of host memory that the
 // closing workgroup stores: the host follows the run without a copy in the
@@ -282,7 +307,8 @@ struct step_core {
   group_stats* gst;     // kTicketGroups partial slots
   unsigned small_grid;  // least grid of a push iteration (0: push iterations use the whole grid)
   unsigned* board;      // completion-ticket counters (kTicketWords)
-  unsigned max_outdeg;  // largest out-degree of the graph (0: unknown)
+  unsigned max_outdeg;  // largest out-degree of the graph (0: see graph_maxdeg)
+  const unsigned* graph_maxdeg;  // device word that holds it, or null
   unsigned persist_edges;  // persist_kernel: largest queue out-edge total it takes (0: off)
   unsigned long long* progress;  // pinned host word (progress_pack), or null
   // Source-split in-CSR for the edge-balanced pull (used when xsplit != 0):
@@ -360,6 +386,7 @@ struct step_smem {
 
 struct iter_ctx {
   unsigned iter;
+  unsigned max_iter, launches;   // from the control line
   unsigned grid;      // workgroups that share this iteration's work (the first `grid`)
   const unsigned long long* in_bm;
   unsigned long long* out_bm;
@@ -371,6 +398,8 @@ struct iter_ctx {
   unsigned in_count;
   unsigned long long in_edges;   // push: out-edges of the input queue (its sentinel offset)
   bool tiny;          // push: entries + out-edges <= kTinyWork (bits claimed without a read)
+  bool few;           // tiny, and no out-list is longer than kFewDegree
+  bool few_close;     // and close_few ends the iteration
   step_stats* st;
   bool scatter;
   bool dense_in;      // the updated set's out-edges cover most edges: pull gathers
@@ -477,9 +506,13 @@ static __global__ void outbits_kernel(const unsigned* __restrict__ oR, unsigned 
   bits[w] = word;
 }
 
-// Largest out-degree: *out = max over v < n of oR[v+1] - oR[v] (*out starts at 0).
+// Largest out-degree: *out = max over v < n of oR[v+1] - oR[v] (*out starts
+// at 0; one atomic per workgroup: they all hit one line).
 static __global__ void max_outdeg_kernel(const unsigned* __restrict__ oR, unsigned n,
                                          unsigned* __restrict__ out) {
+  __shared__ unsigned s_max;
+  if (threadIdx.x == 0) s_max = 0;
+  __syncthreads();
   unsigned const stride = gridDim.x * blockDim.x;
   unsigned md = 0;
   for (unsigned v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
@@ -487,7 +520,9 @@ static __global__ void max_outdeg_kernel(const unsigned* __restrict__ oR, unsign
     md = d > md ? d : md;
   }
   md = wave_max(md);
-  if ((threadIdx.x & 63) == 0 && md) atomicMax(out, md);
+  if ((threadIdx.x & 63) == 0 && md) atomicMax(&s_max, md);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_max) atomicMax(out, s_max);
 }
 
 // ---- native min for the min-semilattice fast path --------------------------
@@ -615,6 +650,32 @@ __device__ __forceinline__ void append_queue(P& p, iter_ctx& c, lane_acc& la, bo
   bool const w[1] = {want};
   unsigned const vv[1] = {v};
   stage_queue(p, c, la, w, vv);
+}
+
+// The same for one vertex per lane whose out-degree the caller holds.
+__device__ __forceinline__ void append_with_degree(iter_ctx& c, lane_acc& la, bool want, unsigned v,
+                                                   unsigned deg) {
+  unsigned long long const m = ballot64(want);
+  if (!m) return;
+  unsigned const tc = static_cast<unsigned>(__builtin_popcountll(m));
+  unsigned const d = want ? deg : 0u;
+  unsigned const idg = wave_incl_scan(d);
+  unsigned const td = readlane(idg, 63);
+  wave_lds_sync();
+  if (c.ahdr[0] + tc > c.acap) wave_flush(c);
+  unsigned const hc = c.ahdr[0], he = c.ahdr[1];
+  if (want) {
+    unsigned const pos = hc + rank_in(m);
+    c.abuf_v[pos] = v;
+    c.abuf_e[pos] = he + idg - d;
+    la.max_deg = d > la.max_deg ? d : la.max_deg;
+  }
+  wave_lds_sync();
+  if (lane_id() == 0) {
+    c.ahdr[0] = hc + tc;
+    c.ahdr[1] = he + td;
+  }
+  wave_lds_sync();
 }
 
 // Writes the calling wave's staged far-pile entries with one global atomic
@@ -1063,6 +1124,69 @@ __device__ void run_push_wave(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm
           newly = claim_next(c, la, dst, cand, far);
       }
       append_queue(p, c, la, newly, dst);
+      if (c.nf) far_append(c, far, dst);
+    }
+  }
+}
+
+// A tiny push iteration on a graph of short out-lists (at most kFewDegree):
+// bound by its chain of dependent reads, not by throughput.  The waves take
+// equal runs of whole queue entries, so no wave searches the queue's offsets
+// for its share (the edge-balanced form's searches and windows are five or six
+// dependent reads), a relaxation is one returning atomic min, and the
+// destination's out-offsets are read beside it.
+// (Figures at kTinyWork.)
+template <class P, class vT>
+__device__ void run_push_few(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
+  unsigned const lane = lane_id(), wib = threadIdx.x >> 6, t = threadIdx.x;
+  unsigned const waves = c.grid * kWaves, wave = blockIdx.x * kWaves + wib;
+  unsigned const per = (c.in_count + waves - 1) / waves;
+  unsigned const first = wave * per;
+  unsigned const last = first + per < c.in_count ? first + per : c.in_count;
+  unsigned* const excl = sm.excl[wib];
+  unsigned* const base = sm.base[wib];
+  vT* const vals = sm.val[wib];
+  for (unsigned k0 = first; k0 < last; k0 += 64) {
+    unsigned const k = k0 + lane;
+    unsigned r0 = 0, deg = 0;
+    vT val{};
+    if (k < last) {
+      unsigned const u = c.in_q[k];
+      val = p.V[u];
+      r0 = p.oR[u];
+      deg = p.oR[u + 1] - r0;
+      la.active += 1;
+    }
+    la.work += deg;
+    unsigned const incl = wave_incl_scan(deg);
+    unsigned const total = readlane(incl, 63);
+    wave_lds_sync();
+    excl[lane] = incl - deg;
+    base[lane] = r0;
+    vals[lane] = val;
+    wave_lds_sync();
+    for (unsigned c0 = 0; c0 < total; c0 += 64) {
+      unsigned const e = c0 + lane;
+      bool newly = false, far = false;
+      unsigned dst = 0, dd = 0;
+      if (e < total) {
+        unsigned const own = owner_search(excl, e);
+        unsigned const idx = base[own] + (e - excl[own]);
+        dst = p.oC[idx];
+        vT const cand = edge_value(p.fn, sm.tmp[t], vals[own], p.oE + idx);
+        unsigned const d0 = p.oR[dst], d1 = p.oR[dst + 1];
+        vT const old = atomic_min_any(p.V + dst, cand);
+        dd = d1 - d0;
+        if (cand < old && dd) {
+          if (is_near(c, cand)) {
+            newly = set_bit_now(c.out_bm, dst);
+          } else {
+            note_far(la, cand);
+            far = set_bit_now(c.far_bm, dst);
+          }
+        }
+      }
+      append_with_degree(c, la, newly, dst, dd);
       if (c.nf) far_append(c, far, dst);
     }
   }
@@ -1785,63 +1909,15 @@ __device__ unsigned choose_variant(P& p, unsigned count, unsigned long long sdeg
   }
 }
 
-template <class P, class vT>
-__device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<vT>& sm) {
-  // Every statistic and queue counter of this workgroup was updated by an
-  // agent-scope atomic whose result has returned (or, for thread 0's own
-  // counter updates, is waited for here) before the ticket is taken, so the
-  // last workgroup reads complete counters without an L2 write-back fence.
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_s_waitcnt(0);
-    sm.is_last = take_ticket(p.board);
-  }
-  __syncthreads();
-  if (!sm.is_last) return;
-  if (threadIdx.x >= 64) return;
+// The end of an iteration whose updated set has `count` queue entries with
+// `sdeg` out-edges (first wave of the last workgroup): the next variant and the
+// control line.
+template <class P>
+__device__ __forceinline__ void close_iteration(P& p, iter_ctx& c, unsigned iter, unsigned count,
+                                                unsigned long long sdeg, bool learned, unsigned ng,
+                                                bool pre_md, unsigned md_part,
+                                                learned_in const& li) {
   step_stats* st = p.stats + iter;
-  bool const learned = p.sched.mode == SCHED_LEARNED;
-  unsigned const ng = gridDim.x < kTicketGroups ? gridDim.x : kTicketGroups;
-  // The queue counter, the iteration limit, the learned schedule's
-  // max-degree partials, decision cache and network weights are all loaded
-  // before any of them is used, so they come back in one round trip (the
-  // fold and the inference would otherwise each start another one on this
-  // serial path).  Both queue counters are read whatever the variant;
-  // lanes past the group count read slot 0 again (max is unchanged).
-  unsigned long long const qe =
-      __hip_atomic_load(&st->qe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  unsigned const scount =
-      __hip_atomic_load(&st->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  unsigned const max_iter = p.ctl->max_iter;
-  bool const pre_md = learned && !c.no_deg && !p.collect && !c.nf;
-  unsigned const md_part =
-      __hip_atomic_load(&p.gst[lane_id() < ng ? lane_id() : 0u].max_deg, __ATOMIC_RELAXED,
-                        __HIP_MEMORY_SCOPE_AGENT);
-  // (no branch between the loads: a run without a network reads the group
-  // slots as its weights, any readable MLP_NPARAM floats, and never uses
-  // them)
-  static_assert(sizeof(group_stats) * kTicketGroups >= sizeof(float) * MLP_NPARAM,
-                "the group slots stand in for absent weights");
-  learned_in li;
-  li.cache_key = p.ctl->cache_key;
-  li.cache_variant = p.ctl->cache_variant;
-  mlp_load_lane(p.sched.mlp ? p.sched.mlp : reinterpret_cast<const float*>(p.gst), li.w);
-  unsigned count;
-  unsigned long long sdeg;
-  if (c.scatter) {
-    count = scount;
-    sdeg = 0;
-  } else {
-    // Queue length and out-edge total from the packed append counter; the
-    // sentinel offset closes the queue's offset array.
-    count = qe_count(qe);
-    sdeg = qe_edges(qe);
-    if (threadIdx.x == 0) {
-      st->count = count;
-      st->sum_outdeg = sdeg;
-      c.out_qe[count] = static_cast<unsigned>(sdeg);
-    }
-  }
   unsigned maxdeg = 0;
   unsigned long long vmin = ~0ull;
   // The learned schedule uses the next frontier's max degree only when its
@@ -1874,7 +1950,7 @@ __device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<v
     split_next = count == 0 && far_n != 0;
   }
   unsigned next = V_CLASSIC;
-  bool const stop = (count == 0 && !split_next) || (iter + 1 >= max_iter);
+  bool const stop = (count == 0 && !split_next) || (iter + 1 >= c.max_iter);
   if (!stop)
     next = split_next ? static_cast<unsigned>(V_SPLIT)
                       : choose_variant(p, count, sdeg, maxdeg, iter + 1, li);
@@ -1900,7 +1976,7 @@ __device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<v
     unsigned const level = stop || iter + 1 < kGrowIters ? 0u
                            : split_next                  ? (far_n <= kSmallWork ? 1u : 0u)
                                                          : grid_level(next, count, sdeg);
-    unsigned const launches = p.ctl->launches + 1;
+    unsigned const launches = c.launches + 1;
     bool const over = stop && (count != 0 || split_next);
     p.ctl->small_next = level;
     p.ctl->launches = launches;
@@ -1913,6 +1989,131 @@ __device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<v
     if (p.progress)
       __hip_atomic_store(p.progress, progress_pack(iter + 1, launches, level, stop, over),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+template <class P, class vT>
+__device__ void finalize_iteration(P& p, iter_ctx& c, unsigned iter, step_smem<vT>& sm) {
+  // Every statistic and queue counter of this workgroup was updated by an
+  // agent-scope atomic whose result has returned (or, for thread 0's own
+  // counter updates, is waited for here) before the ticket is taken, so the
+  // last workgroup reads complete counters without an L2 write-back fence.
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_s_waitcnt(0);
+    sm.is_last = take_ticket(p.board);
+  }
+  __syncthreads();
+  if (!sm.is_last) return;
+  if (threadIdx.x >= 64) return;
+  step_stats* st = p.stats + iter;
+  bool const learned = p.sched.mode == SCHED_LEARNED;
+  unsigned const ng = gridDim.x < kTicketGroups ? gridDim.x : kTicketGroups;
+  // The queue counter, the learned schedule's max-degree partials, decision cache and network weights are all loaded
+  // before any of them is used, so they come back in one round trip (the
+  // fold and the inference would otherwise each start another one on this
+  // serial path).  Both queue counters are read whatever the variant;
+  // lanes past the group count read slot 0 again (max is unchanged).
+  unsigned long long const qe =
+      __hip_atomic_load(&st->qe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned const scount =
+      __hip_atomic_load(&st->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  bool const pre_md = learned && !c.no_deg && !p.collect && !c.nf;
+  unsigned const md_part =
+      __hip_atomic_load(&p.gst[lane_id() < ng ? lane_id() : 0u].max_deg, __ATOMIC_RELAXED,
+                        __HIP_MEMORY_SCOPE_AGENT);
+  // (no branch between the loads: a run without a network reads the group
+  // slots as its weights, any readable MLP_NPARAM floats, and never uses
+  // them)
+  static_assert(sizeof(group_stats) * kTicketGroups >= sizeof(float) * MLP_NPARAM,
+                "the group slots stand in for absent weights");
+  learned_in li;
+  li.cache_key = p.ctl->cache_key;
+  li.cache_variant = p.ctl->cache_variant;
+  mlp_load_lane(p.sched.mlp ? p.sched.mlp : reinterpret_cast<const float*>(p.gst), li.w);
+  unsigned count;
+  unsigned long long sdeg;
+  if (c.scatter) {
+    count = scount;
+    sdeg = 0;
+  } else {
+    // Queue length and out-edge total from the packed append counter; the
+    // sentinel offset closes the queue's offset array.
+    count = qe_count(qe);
+    sdeg = qe_edges(qe);
+    if (threadIdx.x == 0) {
+      st->count = count;
+      st->sum_outdeg = sdeg;
+      c.out_qe[count] = static_cast<unsigned>(sdeg);
+    }
+  }
+  close_iteration(p, c, iter, count, sdeg, learned, ng, pre_md, md_part, li);
+}
+
+// Closes a tiny iteration of run_push_few on a grid of at most kFewGrid
+// workgroups: one returning atomic per workgroup reserves its queue slots and
+// out-edge offsets and counts it in, and hands the last one the totals (the
+// general close takes a queue atomic, a ticket and a read of the totals one
+// after the other).  Everything else a workgroup wrote is ordered by the end of
+// the launch.  Whole workgroup.
+template <class P, class vT>
+__device__ void close_few(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm) {
+  if (c.nf) flush_stats(sm, la, false, true);
+  __syncthreads();
+  unsigned const wib = threadIdx.x >> 6, lane = lane_id();
+  unsigned const ng = gridDim.x < kTicketGroups ? gridDim.x : kTicketGroups;
+  if (threadIdx.x == 0) {
+    unsigned tc = 0, te = 0;
+    for (int w = 0; w < kWaves; ++w) {
+      tc += sm.ahdr[w][0];
+      te += sm.ahdr[w][1];
+    }
+    if (c.nf) {
+      unsigned tf = 0;
+      for (int w = 0; w < kWaves; ++w) tf += sm.ahdr[w][2];
+      unsigned long long r = 0;
+      if (sm.bvmin != ~0ull) r = atomicMin(&p.gst[blockIdx.x % ng].vmin, sm.bvmin);
+      sm.fbase = tf ? atomicAdd(c.far_n, tf) : 0u;
+      keep_live(r);
+      __builtin_amdgcn_s_waitcnt(0);
+    }
+    unsigned long long const old = atomicAdd(&p.ctl->few, few_pack(1u, tc, te));
+    sm.bbase = old;
+    sm.is_last = static_cast<unsigned>(old >> 56) == gridDim.x - 1;
+  }
+  __syncthreads();
+  unsigned long long const old = sm.bbase;
+  unsigned bc = few_count(old), be = static_cast<unsigned>(old);
+  for (unsigned w = 0; w < wib; ++w) {
+    bc += sm.ahdr[w][0];
+    be += sm.ahdr[w][1];
+  }
+  unsigned const cnt = sm.ahdr[wib][0];
+  for (unsigned i = lane; i < cnt; i += WAVE_SIZE) {
+    c.out_q[bc + i] = sm.abuf_v[wib][i];
+    c.out_qe[bc + i] = be + sm.abuf_e[wib][i];
+  }
+  if (c.nf) {
+    unsigned fb = sm.fbase;
+    for (unsigned w = 0; w < wib; ++w) fb += sm.ahdr[w][2];
+    unsigned const fc = sm.ahdr[wib][2];
+    for (unsigned i = lane; i < fc; i += WAVE_SIZE) c.far_q[fb + i] = c.fbuf[i];
+  }
+  if (sm.is_last && threadIdx.x < 64) {
+    unsigned count = few_count(old), edges = static_cast<unsigned>(old);
+    for (int w = 0; w < kWaves; ++w) {
+      count += sm.ahdr[w][0];
+      edges += sm.ahdr[w][1];
+    }
+    if (threadIdx.x == 0) {
+      p.ctl->few = 0ull;
+      c.st->qe = qe_pack(count, edges);
+      c.st->count = count;
+      c.st->sum_outdeg = edges;
+      c.out_qe[count] = edges;
+    }
+    close_iteration(p, c, c.iter, count, edges, p.sched.mode == SCHED_LEARNED, ng, false, 0u,
+                    learned_in{});
   }
 }
 
@@ -1929,6 +2130,8 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
   unsigned const variant = p.ctl->next_variant;
   iter_ctx c;
   c.iter = iter;
+  c.max_iter = p.ctl->max_iter;
+  c.launches = p.ctl->launches;
   unsigned long long const nw = p.nwords;
   c.in_bm = p.bm + (iter % 3) * nw;
   c.out_bm = p.bm + ((iter + 1) % 3) * nw;
@@ -1950,6 +2153,8 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
   }
   c.in_edges = in_edges;
   c.tiny = static_cast<unsigned long long>(c.in_count) + in_edges <= kTinyWork;
+  unsigned const max_outdeg = p.ctl->max_outdeg;
+  c.few = c.tiny && max_outdeg != 0 && max_outdeg <= kFewDegree;
   c.dense_in = iter > 0 && in_edges * 10ull >= p.m * 7ull;
   // The split pays where the pull gathers much (the updated set's out-edges
   // cover a quarter of the edges or more); on a sparse pull its extra
@@ -1964,8 +2169,8 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
   // Settled runs never infer (they take the plain rule): no statistics.
   c.no_deg = p.sched.mode == SCHED_LEARNED && !p.collect && !(NF && MIN_FAST) &&
              (p.sched.settled_below != 0 ||
-              (iter > 0 && p.max_outdeg != 0 && variant >= V_PUSH_T && variant <= V_PUSH_LB &&
-               in_edges <= kSmallWork / (1ull + p.max_outdeg)));
+              (iter > 0 && max_outdeg != 0 && variant >= V_PUSH_T && variant <= V_PUSH_LB &&
+               in_edges <= kSmallWork / (1ull + max_outdeg)));
   c.variant = variant;
   c.nf = false;
   c.T = ~0ull;
@@ -2018,6 +2223,16 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
   c.ahdr = sm.ahdr[wib];
   c.acap = c.nf ? kAcap / 2 : kAcap;
   c.fbuf = sm.abuf_v[wib] + kAcap / 2;
+  // close_few counts entries apart from the statistics' append counter, so no
+  // wave may flush its staging buffer before: a wave's entries are bounded by
+  // its share of the queue times the largest out-degree.
+  c.few_close = false;
+  if constexpr (DELTA && MIN_FAST) {
+    unsigned const waves = c.grid * kWaves;
+    c.few_close = c.few && variant == V_PUSH_LB && gridDim.x <= kFewGrid && !p.collect &&
+                  ((c.in_count + waves - 1) / waves) * max_outdeg <= c.acap &&
+                  (p.sched.mode != SCHED_LEARNED || c.no_deg);
+  }
   if ((threadIdx.x & 63) == 0) {
     sm.ahdr[wib][0] = 0;
     sm.ahdr[wib][1] = 0;
@@ -2039,7 +2254,15 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
       case V_PUSH_W: run_push_wave<MIN_FAST>(p, c, la, sm); break;
       case V_PUSH_B: run_push_block<MIN_FAST>(p, c, la, sm); break;
       case V_PULL_T: run_pull_thread<MIN_FAST>(p, c, la, sm); break;
-      case V_PUSH_LB: run_lb<LB_PUSH, MIN_FAST>(p, c, la, sm); break;
+      case V_PUSH_LB:
+        if constexpr (MIN_FAST) {
+          if (c.few) {
+            run_push_few(p, c, la, sm);
+            break;
+          }
+        }
+        run_lb<LB_PUSH, MIN_FAST>(p, c, la, sm);
+        break;
       case V_PULL_W: run_pull_wave<MIN_FAST>(p, c, la, sm); break;
       case V_PULL_B: run_pull_block<MIN_FAST>(p, c, la, sm); break;
       case V_PULL_LB: run_lb<LB_PULL, MIN_FAST>(p, c, la, sm); break;
@@ -2050,6 +2273,17 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
     }
   } else {
     run_classic<false>(p, c, la, sm);
+  }
+  if (c.few_close) {
+    close_few(p, c, la, sm);
+    for (unsigned w = blockIdx.x * blockDim.x + threadIdx.x; w < p.nwords;
+         w += gridDim.x * blockDim.x)
+      c.clr_bm[w] = 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      c.st->variant = variant;
+      c.st->in_count = c.in_count;
+    }
+    return;
   }
   if (!idle) {
     bool const want_stats =
@@ -2147,6 +2381,8 @@ __global__ void start_kernel(P p, unsigned nstats, unsigned first_variant, unsig
     ctl->seed_count = count;
     ctl->small_next = 0;
     ctl->launches = 0;
+    ctl->few = 0;
+    ctl->max_outdeg = p.max_outdeg ? p.max_outdeg : p.graph_maxdeg ? *p.graph_maxdeg : 0u;
     ctl->q_count = 0;
     ctl->q_edges = 0;
     ctl->cache_key = 0xffffffffu;

@@ -737,7 +737,7 @@ namespace detail {
 inline unsigned max_outdeg_into(unsigned* w, const unsigned* oR, std::size_t nv, stream& s) {
   hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s.get(), w, 1u);
   if (nv) {
-    unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 255) / 256, 4096));
+    unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 1023) / 1024, 512));
     hipLaunchKernelGGL(max_outdeg_kernel, dim3(blocks), dim3(256), 0, s.get(), oR,
                        static_cast<unsigned>(nv), w);
   }
@@ -842,9 +842,10 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
                                           offsetof(step_ctl, board));
   prm.small_grid = o.adaptive_grid ? small_grid_of(dev, o) : 0u;
   prm.persist_edges = o.persist ? std::min(o.persist_edges, detail::kPersistEdges) : 0u;
-  if (sch == schedule::learned)
-    prm.max_outdeg = ws ? ws->max_outdeg_of(grph.oR.get_ptr(), n, s)
-                        : max_outdeg_into(st.word, grph.oR.get_ptr(), n, s);
+  if (ws && sch != schedule::classic)
+    prm.graph_maxdeg = ws->maxdeg_of(grph.oR.get_ptr(), n, s);
+  else if (sch == schedule::learned)
+    prm.max_outdeg = max_outdeg_into(st.word, grph.oR.get_ptr(), n, s);
   if (o.split_pull && sch != schedule::classic) {
     ensure_split(grph, s);
     prm.xsplit = 1u;

@@ -122,26 +122,21 @@ struct workspace {
   launch_cache graphs;                     // captured iteration chunks
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the two control-line copies in flight
-  unsigned max_outdeg = 0;                 // the graph's largest out-degree, once computed
-  bool have_max_outdeg = false;
+  device_buffer<unsigned> maxdeg;          // the graph's largest out-degree
 
-  // Largest out-degree of the graph whose out-offsets are oR (n vertices),
-  // computed on the device the first time and kept.
-  unsigned max_outdeg_of(const unsigned* oR, std::size_t nv, stream& s) {
-    if (have_max_outdeg) return max_outdeg;
-    device_buffer<unsigned> out(1, dev);
-    KITES_HIP_CHECK(hipMemsetAsync(out.get_ptr(), 0, sizeof(unsigned), s.get()));
+  // Device word with the largest out-degree of the graph whose out-offsets are
+  // oR (n vertices), computed on `s` the first time and kept.
+  const unsigned* maxdeg_of(const unsigned* oR, std::size_t nv, stream& s) {
+    if (maxdeg.size()) return maxdeg.get_ptr();
+    maxdeg.alloc(1, dev);
+    hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s.get(), maxdeg.get_ptr(), 1u);
     if (nv) {
-      unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 255) / 256, 4096));
+      unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 1023) / 1024, 512));
       hipLaunchKernelGGL(max_outdeg_kernel, dim3(blocks), dim3(256), 0, s.get(), oR,
-                         static_cast<unsigned>(nv), out.get_ptr());
-      KITES_HIP_CHECK(hipPeekAtLastError());
+                         static_cast<unsigned>(nv), maxdeg.get_ptr());
     }
-    KITES_HIP_CHECK(hipMemcpyAsync(&max_outdeg, out.get_ptr(), sizeof(unsigned),
-                                   hipMemcpyDeviceToHost, s.get()));
-    s.sync();
-    have_max_outdeg = true;
-    return max_outdeg;
+    KITES_HIP_CHECK(hipPeekAtLastError());
+    return maxdeg.get_ptr();
   }
 
   void ensure(std::size_t nv, unsigned iters, int device) {
