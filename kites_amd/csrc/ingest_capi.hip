@@ -28,16 +28,22 @@ int kites_graph_from_edges(int32_t device, uint32_t n, uint64_t m, const uint32_
   std::unique_ptr<kites_graph> g(new kites_graph());
   g->dev.reset(new kites::gpu(device));
   int const did = g->dev->getDevIdx();
-  kites::device_buffer<unsigned> ds(m ? m : 1, did), dd(m ? m : 1, did), dw(m ? m : 1, did);
+  kites::device_arena edges;
+  unsigned *ds = nullptr, *dd = nullptr, *dw = nullptr;
+  edges.begin();
+  edges.add(ds, m ? m : 1);
+  edges.add(dd, m ? m : 1);
+  edges.add(dw, m ? m : 1);
+  edges.commit(did);
   if (m) {
-    KITES_HIP_CHECK(hipMemcpy(ds.get_ptr(), src, m * 4, hipMemcpyHostToDevice));
-    KITES_HIP_CHECK(hipMemcpy(dd.get_ptr(), dst, m * 4, hipMemcpyHostToDevice));
-    KITES_HIP_CHECK(hipMemcpy(dw.get_ptr(), w, m * 4, hipMemcpyHostToDevice));
+    KITES_HIP_CHECK(hipMemcpy(ds, src, m * 4, hipMemcpyHostToDevice));
+    KITES_HIP_CHECK(hipMemcpy(dd, dst, m * 4, hipMemcpyHostToDevice));
+    KITES_HIP_CHECK(hipMemcpy(dw, w, m * 4, hipMemcpyHostToDevice));
   }
   kites::ingest_report rep;
   g->g.reset(new kites::graph_csr_device<unsigned, unsigned>(
       kites::make_graph_csr_from_edges<unsigned, unsigned, unsigned>(
-          *g->dev, n, m, ds.get_ptr(), dd.get_ptr(), dw.get_ptr(), dedup != 0, &rep)));
+          *g->dev, n, m, ds, dd, dw, dedup != 0, &rep)));
   g->n = static_cast<uint32_t>(rep.n);
   g->m = rep.m;
   if (build_ms) *build_ms = rep.build_ms;

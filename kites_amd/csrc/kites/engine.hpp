@@ -621,17 +621,17 @@ void run_ordered(ordered_view<vT, eT> const& g, gpu& dev, stream& s, ordered_wor
   prm.V = g.V;
   prm.nwords = nwords;
   prm.ntasks = ntasks;
-  ws.begin();
-  ws.add(prm.W, n);
-  ws.add(prm.bm, 2 * static_cast<std::size_t>(nwords));
-  ws.add(prm.hasin, nwords);
-  ws.add(prm.tstart, static_cast<std::size_t>(ntasks) + 1);
-  ws.add(prm.hv, hcap);
-  ws.add(prm.hbase, hcap);
-  ws.add(prm.hact, hcap);
-  ws.add(prm.hchunk, ccap);
-  ws.add(prm.hsum, ccap);
-  ws.add(prm.ctl, 1);
+  ws.mem.begin();
+  ws.mem.add(prm.W, n);
+  ws.mem.add(prm.bm, 2 * static_cast<std::size_t>(nwords));
+  ws.mem.add(prm.hasin, nwords);
+  ws.mem.add(prm.tstart, static_cast<std::size_t>(ntasks) + 1);
+  ws.mem.add(prm.hv, hcap);
+  ws.mem.add(prm.hbase, hcap);
+  ws.mem.add(prm.hact, hcap);
+  ws.mem.add(prm.hchunk, ccap);
+  ws.mem.add(prm.hsum, ccap);
+  ws.mem.add(prm.ctl, 1);
   ws.commit(dev.getDevIdx());
   KITES_HIP_CHECK(hipEventRecord(ws.ev0, s.get()));
   unsigned const max_iter = std::max(1u, o.max_iterations);

@@ -68,33 +68,17 @@ struct batch_workspace {
   }
 };
 
-// Device state of ordered runs: one allocation, kept between runs and grown
-// when a run needs more, cut into the run's arrays (add() each, then commit()).
+// Device state of ordered runs (an arena, kept between runs).
 struct ordered_workspace {
-  device_buffer<unsigned char> mem;
+  device_arena mem;
   host_pinned_buffer<ordered_ctl> host;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  std::vector<std::pair<unsigned char**, std::size_t>> parts;
-  std::size_t bytes = 0;
 
-  void begin() {
-    parts.clear();
-    bytes = 0;
-  }
-  template <class T>
-  void add(T*& p, std::size_t count) {
-    parts.emplace_back(reinterpret_cast<unsigned char**>(&p), bytes);
-    bytes += (count * sizeof(T) + 255) & ~std::size_t(255);
-  }
   void commit(int dev) {
-    if (mem.size() < bytes) {
-      mem.free();
-      mem.alloc(bytes, dev);
-    }
+    mem.commit(dev);
     if (host.size() == 0) host.alloc(1);
     if (!ev0) KITES_HIP_CHECK(hipEventCreate(&ev0));
     if (!ev1) KITES_HIP_CHECK(hipEventCreate(&ev1));
-    for (auto const& x : parts) *x.first = mem.get_ptr() + x.second;
   }
   ~ordered_workspace() {
     if (ev0) (void)hipEventDestroy(ev0);
@@ -108,6 +92,7 @@ struct workspace {
   std::size_t n = 0;
   unsigned nwords = 0;
   unsigned max_iter = 0;
+  device_arena arena;                     // the run state but the far piles
   device_buffer<unsigned long long> bm;   // 3 bitmaps of nwords words
   device_buffer<unsigned> q;              // 2 queues of n entries
   device_buffer<unsigned> qe;             // 2 offset arrays of n + 1 entries
@@ -123,12 +108,13 @@ struct workspace {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the two control-line copies in flight
   device_buffer<unsigned> maxdeg;          // the graph's largest out-degree
+  bool have_maxdeg = false;
 
   // Device word with the largest out-degree of the graph whose out-offsets are
   // oR (n vertices), computed on `s` the first time and kept.
   const unsigned* maxdeg_of(const unsigned* oR, std::size_t nv, stream& s) {
-    if (maxdeg.size()) return maxdeg.get_ptr();
-    maxdeg.alloc(1, dev);
+    if (have_maxdeg) return maxdeg.get_ptr();
+    have_maxdeg = true;
     hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s.get(), maxdeg.get_ptr(), 1u);
     if (nv) {
       unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 1023) / 1024, 512));
@@ -142,27 +128,30 @@ struct workspace {
   void ensure(std::size_t nv, unsigned iters, int device) {
     dev = device;
     unsigned const words = static_cast<unsigned>((nv + 63) / 64 + 1);
-    if (nv > n || words > nwords) {
-      bm.free();
-      bm.alloc(3ull * words, dev);
-      q.free();
-      q.alloc(2 * (nv ? nv : 1), dev);
-      qe.free();
-      qe.alloc(2 * (nv + 1), dev);
-      fq.free();
-      fbm.free();
-      n = nv;
-      nwords = words;
+    if (nv > n || words > nwords || iters > max_iter || ctl.size() == 0) {
+      if (nv > n || words > nwords) {
+        fq.free();
+        fbm.free();
+      }
+      std::size_t const cap = std::max(nv, n);
+      unsigned const capw = std::max(words, nwords), capi = std::max(iters, max_iter);
+      n = nwords = max_iter = 0;   // (planned again if the allocation fails)
+      arena.begin();
+      arena.add(bm, 3ull * capw, dev);
+      arena.add(q, 2 * (cap ? cap : 1), dev);
+      arena.add(qe, 2 * (cap + 1), dev);
+      arena.add(stats, capi, dev);
+      arena.add(ctl, 1, dev);
+      arena.add(gst, kTicketGroups, dev);
+      arena.add(maxdeg, 1, dev);
+      arena.commit(dev);
+      n = cap;
+      nwords = capw;
+      max_iter = capi;
+      have_maxdeg = false;
     }
-    if (iters > max_iter) {
-      stats.free();
-      stats.alloc(iters, dev);
-      max_iter = iters;
-    }
-    if (ctl.size() == 0) {
-      ctl.alloc(1, dev);
+    if (ctl_host.size() == 0) {
       ctl_host.alloc(2);
-      gst.alloc(kTicketGroups, dev);
       KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&progress), sizeof(unsigned long long),
                                     hipHostMallocPortable | hipHostMallocCoherent));
       // (start_kernel writes all of the control block that a run reads, on the
@@ -235,6 +224,7 @@ class graph_csr_device : public graph_base {
 
  public:
   int residing_device_id;
+  device_arena vertex_arena, edge_arena;   // graphs built from edges: their arrays' memory
   device_buffer<vT> V;
   device_buffer<eIdxT> R;
   device_buffer<vIdxT> C;
@@ -284,7 +274,7 @@ class graph_csr_device : public graph_base {
   device_buffer<unsigned long long> outbits;
   void build_outbits(std::size_t n, stream& s) {
     unsigned const nw = static_cast<unsigned>((n + 63) / 64 + 1);
-    outbits.alloc(nw, residing_device_id);
+    outbits.alloc(nw, residing_device_id);   // (no-op if the arena holds it)
     hipLaunchKernelGGL(detail::outbits_kernel, dim3((nw + 255) / 256), dim3(256), 0, s.get(),
                        oR.get_ptr(), static_cast<unsigned>(n), outbits.get_ptr(), nw);
     KITES_HIP_CHECK(hipPeekAtLastError());
@@ -364,15 +354,18 @@ class graph_csr_device : public graph_base {
           dev.setAsActive();
           return dev.getDevIdx();
         }()},
-        V{n, residing_device_id},
-        R{n + 1, residing_device_id},
-        vBitmapEven{n, residing_device_id},
-        vBitmapOdd{n, residing_device_id},
-        updateFlag{1, residing_device_id},
         updateFlagHost{1},
         gProp{graph_property::directed},
-        vertexPerGroup{1},
-        oR{n + 1, residing_device_id} {
+        vertexPerGroup{1} {
+    vertex_arena.begin();
+    vertex_arena.add(V, n, residing_device_id);
+    vertex_arena.add(R, n + 1, residing_device_id);
+    vertex_arena.add(oR, n + 1, residing_device_id);
+    vertex_arena.add(vBitmapEven, n, residing_device_id);
+    vertex_arena.add(vBitmapOdd, n, residing_device_id);
+    vertex_arena.add(updateFlag, 1, residing_device_id);
+    vertex_arena.add(outbits, (n + 63) / 64 + 1, residing_device_id);
+    vertex_arena.commit(residing_device_id);
     stream& s = dev.getSsEven();
     KITES_HIP_CHECK(hipMemsetAsync(V.get_ptr(), 0, n * sizeof(vT), s.get()));
     KITES_HIP_CHECK(hipMemsetAsync(vBitmapEven.get_ptr(), 0, vBitmapEven.sizeInBytes(), s.get()));

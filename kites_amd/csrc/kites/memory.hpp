@@ -15,7 +15,10 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <functional>
 #include <iostream>
+#include <utility>
+#include <vector>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -125,6 +128,7 @@ class host_bitmap : public host_pinned_buffer<unsigned int> {
 template <typename T>
 class device_buffer : public uva_buffer<T> {
   int residing_device_id;
+  bool adopted = false;   // a part of a device_arena: not freed here
 
   void construct(std::size_t n) {
     KITES_HIP_CHECK(hipSetDevice(residing_device_id));
@@ -136,9 +140,20 @@ class device_buffer : public uva_buffer<T> {
   void free() override {
     if (this->nElems != 0) {
       this->nElems = 0;
-      KITES_HIP_CHECK(hipFree(this->ptr));
+      T* const p = this->ptr;
       this->ptr = nullptr;
+      if (!adopted) KITES_HIP_CHECK(hipFree(p));
+      adopted = false;
     }
+  }
+  // Takes n values at p, memory that another object owns and outlives this one
+  // (device_arena).
+  void adopt(T* p, std::size_t n, int dev) {
+    free();
+    residing_device_id = dev;
+    this->ptr = n ? p : nullptr;
+    this->nElems = n;
+    adopted = n != 0;
   }
   device_buffer() : residing_device_id{0} {}
   device_buffer(std::size_t n, int dev) : residing_device_id{dev} {
@@ -152,9 +167,12 @@ class device_buffer : public uva_buffer<T> {
   }
   device_buffer& operator=(device_buffer const&) = delete;
   device_buffer(device_buffer&& in)
-      : uva_buffer<T>{in.size(), in.get_ptr()}, residing_device_id{in.residing_device_id} {
+      : uva_buffer<T>{in.size(), in.get_ptr()},
+        residing_device_id{in.residing_device_id},
+        adopted{in.adopted} {
     in.nElems = 0;
     in.ptr = nullptr;
+    in.adopted = false;
   }
   device_buffer& operator=(device_buffer&& in) {
     if (this != &in) {
@@ -162,8 +180,10 @@ class device_buffer : public uva_buffer<T> {
       this->nElems = in.nElems;
       this->ptr = in.ptr;
       residing_device_id = in.residing_device_id;
+      adopted = in.adopted;
       in.nElems = 0;
       in.ptr = nullptr;
+      in.adopted = false;
     }
     return *this;
   }
@@ -197,7 +217,57 @@ class device_bitmap : public device_buffer<unsigned long long> {
     if (n > 0) nBits = n;
     device_buffer<unsigned long long>::alloc((n + 63) / 64 + 1, dev);
   }
+  void adopt(unsigned long long* p, std::size_t n, int dev) {
+    nBits = n;
+    device_buffer<unsigned long long>::adopt(p, (n + 63) / 64 + 1, dev);
+  }
   std::size_t getnBits() const { return nBits; }
+};
+
+// Several arrays in one device allocation (hipMalloc costs about 55 us and
+// hipFree 185 us apiece: a graph and its run state are some twenty arrays).
+// add() every array, then commit(); the memory is kept, and grown when a later
+// plan needs more.  The arrays do not outlive the arena.
+class device_arena {
+  device_buffer<unsigned char> mem;
+  std::vector<std::pair<std::size_t, std::function<void(unsigned char*)>>> parts;
+  std::size_t bytes = 0;
+
+  std::size_t place(std::size_t count) {
+    std::size_t const at = bytes;
+    bytes += (count + 255) & ~std::size_t(255);
+    return at;
+  }
+
+ public:
+  void begin() {
+    parts.clear();
+    bytes = 0;
+  }
+  template <class T>
+  void add(T*& p, std::size_t count) {
+    parts.emplace_back(place(count * sizeof(T)),
+                       [&p](unsigned char* at) { p = reinterpret_cast<T*>(at); });
+  }
+  template <class T>
+  void add(device_buffer<T>& b, std::size_t count, int dev) {
+    parts.emplace_back(place(count * sizeof(T)), [&b, count, dev](unsigned char* at) {
+      b.adopt(reinterpret_cast<T*>(at), count, dev);
+    });
+  }
+  void add(device_bitmap& b, std::size_t nbits, int dev) {
+    parts.emplace_back(place(((nbits + 63) / 64 + 1) * 8), [&b, nbits, dev](unsigned char* at) {
+      b.adopt(reinterpret_cast<unsigned long long*>(at), nbits, dev);
+    });
+  }
+  void commit(int dev) {
+    if (mem.size() < bytes) {
+      mem.free();
+      mem.alloc(bytes, dev);
+    }
+    for (auto const& x : parts) x.second(mem.get_ptr() + x.first);
+    parts.clear();
+  }
 };
 
 // ---- copies (mem_ops.cuh:16-88) -------------------------------------------

@@ -132,7 +132,7 @@ void ensure_split(graph_csr_device<vT, eT, vIdxT>& g, stream& s) {
   unsigned const nb = id_bits(n);
   unsigned const mm = static_cast<unsigned>(m);
   device_buffer<unsigned> keyA(m, did), keyB(m, did), valA(m, did), valB(m, did);
-  scratch_bytes tmp;
+  device_buffer<unsigned char> tmp, tmp2;
   hipLaunchKernelGGL(split_keys_kernel, dim3(ingest_grid(m)), dim3(kIngestBlock), 0, s.get(),
                      reinterpret_cast<const unsigned*>(g.R.get_ptr()), static_cast<unsigned>(n),
                      reinterpret_cast<const unsigned*>(g.C.get_ptr()), mm, nb, keyA.get_ptr(),
@@ -143,8 +143,8 @@ void ensure_split(graph_csr_device<vT, eT, vIdxT>& g, stream& s) {
   KITES_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keyA.get_ptr(), keyB.get_ptr(),
                                                      valA.get_ptr(), valB.get_ptr(), m, 0, bits,
                                                      s.get()));
-  tmp.ensure(tb);
-  KITES_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, keyA.get_ptr(), keyB.get_ptr(),
+  tmp.alloc(tb, did);
+  KITES_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp.get_ptr(), tb, keyA.get_ptr(), keyB.get_ptr(),
                                                      valA.get_ptr(), valB.get_ptr(), m, 0, bits,
                                                      s.get()));
   g.xC.alloc(m, did);
@@ -157,8 +157,8 @@ void ensure_split(graph_csr_device<vT, eT, vIdxT>& g, stream& s) {
                      reinterpret_cast<unsigned*>(g.xC.get_ptr()), g.xE.get_ptr(), head);
   KITES_HIP_CHECK(hipPeekAtLastError());
   KITES_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, head, pos, m, s.get()));
-  tmp.ensure(tb);
-  KITES_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, head, pos, m, s.get()));
+  tmp2.alloc(tb, did);
+  KITES_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(tmp2.get_ptr(), tb, head, pos, m, s.get()));
   unsigned last[2] = {0, 0};
   KITES_HIP_CHECK(hipMemcpyAsync(&last[0], pos + (m - 1), 4, hipMemcpyDeviceToHost, s.get()));
   KITES_HIP_CHECK(hipMemcpyAsync(&last[1], head + (m - 1), 4, hipMemcpyDeviceToHost, s.get()));
