@@ -89,7 +89,7 @@ typedef struct kites_run_opts {
                                launch in one workgroup (near-far runs too: far-pile appends
                                and splits of up to twice the limit); plain and learned
                                schedules of SSSP, BFS, CC and SSSP_WRAP.  0: off.  Above 1:
-                               that out-edge limit (at most 16,384). */
+                               that out-edge limit (at most 4,096). */
   int32_t small_grid;       /* workgroups of the launches that follow a small push frontier
                                (entries + out-edges <= 2^18; 0 = one per compute unit) */
   int32_t tiny_grid;        /* ... and a tiny one (<= 2^16; 0 = a quarter of small_grid's
