@@ -236,9 +236,7 @@ struct run_state {
   unsigned* word = nullptr;          // one device word for the largest out-degree (no workspace)
   unsigned nwords = 0;
   unsigned max_iter = 0;
-  step_ctl* ctl_host = nullptr;      // host memory the control header is copied into (two
-                                     // slots when evc is set, else one)
-  hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the copy into each slot (pipelining)
+  step_ctl* ctl_host = nullptr;      // host memory the control header is copied into
   unsigned long long* progress = nullptr;  // pinned word the device reports to (null: copies of
                                            // the control line)
   launch_cache* graphs = nullptr;    // null: iteration chunks are launched directly
@@ -257,12 +255,10 @@ inline run_state state_of(workspace& ws) {
   st.gst = ws.gst.get_ptr();
   st.nwords = ws.nwords;
   st.max_iter = ws.max_iter;
-  st.ctl_host = ws.ctl_host.get_ptr();
+  st.ctl_host = ws.ctl_host;
   st.graphs = &ws.graphs;
   st.ev0 = ws.ev0;
   st.ev1 = ws.ev1;
-  st.evc[0] = ws.evc[0];
-  st.evc[1] = ws.evc[1];
   st.progress = ws.progress;
   return st;
 }
@@ -494,7 +490,7 @@ unsigned record_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options c
                                    s.get()));
   };
   for (;;) {
-    KITES_HIP_CHECK(hipMemcpyAsync(ws.ctl_host.get_ptr(), prm.ctl, offsetof(step_ctl, board),
+    KITES_HIP_CHECK(hipMemcpyAsync(ws.ctl_host, prm.ctl, offsetof(step_ctl, board),
                                    hipMemcpyDeviceToHost, s.get()));
     s.sync();
     step_ctl const ctl = ws.ctl_host[0];
@@ -548,7 +544,7 @@ unsigned record_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options c
           // rollout: replay chunks of forced launches until the run ends;
           // each chunk is timed on its own so host checks add nothing
           for (unsigned k = 0; rv && k <= ws.max_iter / kRollChunk + 1; ++k) {
-            KITES_HIP_CHECK(hipMemcpyAsync(ws.ctl_host.get_ptr(), prm.ctl, offsetof(step_ctl, board),
+            KITES_HIP_CHECK(hipMemcpyAsync(ws.ctl_host, prm.ctl, offsetof(step_ctl, board),
                                            hipMemcpyDeviceToHost, s.get()));
             s.sync();
             if (ws.ctl_host[0].done) break;

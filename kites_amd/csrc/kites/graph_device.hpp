@@ -100,13 +100,12 @@ struct workspace {
   device_buffer<unsigned long long> fbm;  // near-far: far bitmap of nwords words
   device_buffer<step_stats> stats;
   device_buffer<step_ctl> ctl;
-  host_pinned_buffer<step_ctl> ctl_host;
   unsigned long long* progress = nullptr; // pinned host word the closing workgroups store
+  step_ctl* ctl_host = nullptr;           // copies of the control header (same allocation)
   device_buffer<group_stats> gst;         // per-group partial statistics
   ordered_workspace ord;                   // ordered runs (allocated by the first one)
   launch_cache graphs;                     // captured iteration chunks
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipEvent_t evc[2] = {nullptr, nullptr};  // completion of the two control-line copies in flight
   device_buffer<unsigned> maxdeg;          // the graph's largest out-degree
   bool have_maxdeg = false;
 
@@ -150,18 +149,17 @@ struct workspace {
       max_iter = capi;
       have_maxdeg = false;
     }
-    if (ctl_host.size() == 0) {
-      ctl_host.alloc(2);
-      KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&progress), sizeof(unsigned long long),
+    if (!progress) {
+      constexpr std::size_t kWord = 128;
+      KITES_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&progress), kWord + sizeof(step_ctl),
                                     hipHostMallocPortable | hipHostMallocCoherent));
+      ctl_host = reinterpret_cast<step_ctl*>(reinterpret_cast<unsigned char*>(progress) + kWord);
       // (start_kernel writes all of the control block that a run reads, on the
       // run's own stream; a null-stream memset here would not be ordered
       // before it, the stream being a non-blocking one)
-      KITES_HIP_CHECK(hipEventCreate(&ev0));
-      KITES_HIP_CHECK(hipEventCreate(&ev1));
-      KITES_HIP_CHECK(hipEventCreateWithFlags(&evc[0], hipEventDisableTiming));
-      KITES_HIP_CHECK(hipEventCreateWithFlags(&evc[1], hipEventDisableTiming));
     }
+    if (!ev0) KITES_HIP_CHECK(hipEventCreate(&ev0));
+    if (!ev1) KITES_HIP_CHECK(hipEventCreate(&ev1));
   }
   // The near-far far piles and bitmap, allocated by the first run that
   // needs them (after ensure()).
@@ -176,8 +174,6 @@ struct workspace {
     if (progress) (void)hipHostFree(progress);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
-    for (hipEvent_t e : evc)
-      if (e) (void)hipEventDestroy(e);
   }
 };
 

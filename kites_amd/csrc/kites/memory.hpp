@@ -224,48 +224,61 @@ class device_bitmap : public device_buffer<unsigned long long> {
   std::size_t getnBits() const { return nBits; }
 };
 
-// Several arrays in one device allocation (hipMalloc costs about 55 us and
-// hipFree 185 us apiece: a graph and its run state are some twenty arrays).
-// add() every array, then commit(); the memory is kept, and grown when a later
-// plan needs more.  The arrays do not outlive the arena.
+// Several arrays in a few device allocations.  hipMalloc and hipFree of less
+// than 2 MB take 1 us each, larger ones 8 to 125 and 7 to 230 us (a graph and its
+// run state are some twenty arrays): arrays are packed into blocks below that
+// line, and those that reach it share one block.  add() every array, then
+// commit(); the memory is kept, and grown when a later plan needs more.  The
+// arrays do not outlive the arena.
 class device_arena {
-  device_buffer<unsigned char> mem;
-  std::vector<std::pair<std::size_t, std::function<void(unsigned char*)>>> parts;
-  std::size_t bytes = 0;
+  static constexpr std::size_t kBlock = (std::size_t{2} << 20) - 4096;
+  struct part {
+    std::size_t block, at;
+    std::function<void(unsigned char*)> set;
+  };
+  std::vector<device_buffer<unsigned char>> mem;   // block 0: the large arrays
+  std::vector<std::size_t> need;                   // bytes of every block of the plan
+  std::vector<part> parts;
 
-  std::size_t place(std::size_t count) {
-    std::size_t const at = bytes;
-    bytes += (count + 255) & ~std::size_t(255);
-    return at;
+  void place(std::size_t count, std::function<void(unsigned char*)> set) {
+    count = (count + 255) & ~std::size_t(255);
+    std::size_t b = 0;
+    if (count <= kBlock) {
+      if (need.size() == 1 || need.back() + count > kBlock) need.push_back(0);
+      b = need.size() - 1;
+    }
+    parts.push_back({b, need[b], std::move(set)});
+    need[b] += count;
   }
 
  public:
   void begin() {
     parts.clear();
-    bytes = 0;
+    need.assign(1, 0);
   }
   template <class T>
   void add(T*& p, std::size_t count) {
-    parts.emplace_back(place(count * sizeof(T)),
-                       [&p](unsigned char* at) { p = reinterpret_cast<T*>(at); });
+    place(count * sizeof(T), [&p](unsigned char* at) { p = reinterpret_cast<T*>(at); });
   }
   template <class T>
   void add(device_buffer<T>& b, std::size_t count, int dev) {
-    parts.emplace_back(place(count * sizeof(T)), [&b, count, dev](unsigned char* at) {
+    place(count * sizeof(T), [&b, count, dev](unsigned char* at) {
       b.adopt(reinterpret_cast<T*>(at), count, dev);
     });
   }
   void add(device_bitmap& b, std::size_t nbits, int dev) {
-    parts.emplace_back(place(((nbits + 63) / 64 + 1) * 8), [&b, nbits, dev](unsigned char* at) {
+    place(((nbits + 63) / 64 + 1) * 8, [&b, nbits, dev](unsigned char* at) {
       b.adopt(reinterpret_cast<unsigned long long*>(at), nbits, dev);
     });
   }
   void commit(int dev) {
-    if (mem.size() < bytes) {
-      mem.free();
-      mem.alloc(bytes, dev);
-    }
-    for (auto const& x : parts) x.second(mem.get_ptr() + x.first);
+    if (mem.size() < need.size()) mem.resize(need.size());
+    for (std::size_t b = 0; b < need.size(); ++b)
+      if (mem[b].size() < need[b]) {
+        mem[b].free();
+        mem[b].alloc(need[b], dev);
+      }
+    for (auto const& x : parts) x.set(mem[x.block].get_ptr() + x.at);
     parts.clear();
   }
 };
