@@ -70,7 +70,8 @@ typedef struct kites_run_opts {
   int32_t forced_variant;   /* KITES_VAR_* for KITES_SCHED_FORCED */
   float alpha;              /* plain: pull when out-edges(frontier) * alpha > m */
   int32_t use_graph;        /* replay iteration chunks from a captured hipGraph */
-  int32_t chunk;            /* iterations per chunk */
+  int32_t chunk;            /* iterations per chunk (tiny frontiers and small graphs; others
+                               are launched one at a time, a few ahead) */
   int32_t grid;             /* workgroups per launch, 0 = occupancy-derived */
   uint32_t max_iterations;
   int32_t keep_stats;       /* keep per-iteration statistics (kites_graph_stats) */
@@ -85,17 +86,18 @@ typedef struct kites_run_opts {
                                the sources per XCD; one more copy of C and E, built on the
                                first run that sets it); delta schedules only */
   int32_t persist;          /* 1 (default): after a small push frontier, iterations whose
-                               queue fits one workgroup (up to 2,048 out-edges) run many per
-                               launch in one workgroup (near-far runs too: far-pile appends
-                               and splits of up to twice the limit); plain and learned
+                               queue fits one workgroup (up to 2,048 out-edges, near-far
+                               runs 4,096) run many per launch in one workgroup (splits of
+                               up to twice the limit too); plain and learned
                                schedules of SSSP, BFS, CC and SSSP_WRAP.  0: off.  Above 1:
                                that out-edge limit (at most 4,096). */
   int32_t small_grid;       /* workgroups of the launches that follow a small push frontier
                                (entries + out-edges <= 2^18; 0 = one per compute unit) */
   int32_t tiny_grid;        /* ... and a tiny one (<= 2^16; 0 = a quarter of small_grid's
                                default) */
-  int32_t pipeline;         /* 1 (default): after the first chunk of iterations, queue the next
-                               chunk before reading the last one's state; 0: one at a time */
+  int32_t pipeline;         /* 1 (default): follow the run through a word the device stores into
+                               host memory, launches queued ahead; 0: the state is copied back
+                               after every chunk */
 } kites_run_opts;
 
 typedef struct kites_run_info {

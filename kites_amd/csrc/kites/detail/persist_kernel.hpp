@@ -35,8 +35,8 @@
 // 9.2; step_kernel takes 6.2 / 6.5 / 6.9 / 7.0.  Near-far SSSP: 2.8 / 3.0 /
 // 6.1 / 8.5 against 5.9 / 6.4 / 11.1 / 11.9, step_kernel 8.9 / 9.5 / 10.0 /
 // 10.0.  The slope, 2.3 ns per edge, is the unit's scattered accesses, so
-// queues of more than about 2,048 out-edges (the default limit) go to
-// step_kernel: at 4,096 grids of 700 to 2,000 columns take 7.5 to 9.4.
+// BFS queues of more than about 2,048 out-edges go to step_kernel: at 4,096
+// grids of 700 to 2,000 columns take 7.5 to 9.4.
 //
 // The queues are written to memory as step_kernel writes them (queue slot
 // j & 1, offsets, the statistics entry j), the bitmap bits of a queue only when
@@ -80,7 +80,13 @@ constexpr unsigned kPersistRounds = 4;    // edges (or pile entries) per thread
 // Largest out-edge total of a queue it takes (step_core::persist_edges
 // sets the run's limit, at most this): what the two lists in LDS hold.
 constexpr unsigned kPersistEdges = kPersistBlock * kPersistRounds;
+// Default limits.  A step_kernel iteration is 2 to 3 us dearer in near-far runs
+// (two more counters to settle before it can close), so the loop pays for
+// larger queues there: near-far SSSP on grids of 256 / 480 / 700 / 1111 / 2000
+// columns takes 7.8 / 8.5 / 8.5 / 8.9 / 9.0 us per iteration with 2,048 and
+// 6.0 / 8.4 / 8.8 / 8.5 / 8.5 with 4,096.
 constexpr unsigned kPersistDefaultEdges = 2048;
+constexpr unsigned kPersistFarEdges = 4096;
 // Out-lists up to this long are written to the edge list by the lane that
 // appends the vertex, longer ones by its wave.
 constexpr unsigned kPersistLane = 16;

@@ -9,9 +9,11 @@
 //  * No host round trip per iteration.  Each iteration is one launch of
 //    step_kernel; the next iteration's variant, the done flag and the
 //    iteration index are decided on the device by the last workgroup of the
-//    previous launch.  The host replays a captured hipGraph of `chunk`
-//    launches and reads the done flag once per chunk (launches after
-//    convergence return immediately).
+//    previous launch.  The host follows the run through a word the device
+//    stores into pinned host memory and keeps a few launches queued ahead:
+//    single ones on large frontiers, a captured hipGraph of `chunk` launches on
+//    tiny ones and on small graphs (launches after convergence return
+//    immediately).
 //  * The functor set is probed on the host (the lambdas are __host__
 //    __device__).  A set that behaves as a min-semilattice (init copies; red
 //    is idempotent, commutative and associative; upd reports whether red
@@ -101,14 +103,17 @@ struct options {
   bool adaptive_grid = true;             // small grid for chunks of small push frontiers
   unsigned small_grid = 0;               // workgroups of that grid (0 = one per compute unit)
   unsigned tiny_grid = 0;                // after a tiny push frontier (0 = a quarter of those)
-  // After the first chunk, queue the next chunk before reading the last
-  // one's control line (needs the workspace's events; not without).
+  // Follow the run through the progress word the device stores into pinned host
+  // memory and queue launches ahead of it (runs with a workspace; the others,
+  // and all with it off, copy the control line back after every chunk).
   bool pipeline = true;
   // Small push frontiers (min functor sets, plain and learned schedules,
   // near-far too): the chunks that follow a tiny one start with a
   // one-workgroup loop that runs every iteration whose queue fits it
-  // (detail/persist_kernel.hpp) in one launch.  Needs adaptive_grid.  persist_edges: the largest out-edge
-  // total of a queue the loop takes (at most detail::kPersistEdges).
+  // (detail/persist_kernel.hpp) in one launch.  Needs adaptive_grid.
+  // persist_edges: the largest out-edge total of a queue the loop takes (at most
+  // detail::kPersistEdges; left at the default, near-far runs take
+  // detail::kPersistFarEdges).
   bool persist = true;
   unsigned persist_edges = detail::kPersistDefaultEdges;
   // Edge-balanced pull over the source-split in-CSR (split.hpp): each XCD
@@ -837,7 +842,10 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   prm.board = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(st.ctl) +
                                           offsetof(step_ctl, board));
   prm.small_grid = o.adaptive_grid ? small_grid_of(dev, o) : 0u;
-  prm.persist_edges = o.persist ? std::min(o.persist_edges, detail::kPersistEdges) : 0u;
+  unsigned const loop_edges = o.delta && o.persist_edges == detail::kPersistDefaultEdges
+                                  ? detail::kPersistFarEdges
+                                  : o.persist_edges;
+  prm.persist_edges = o.persist ? std::min(loop_edges, detail::kPersistEdges) : 0u;
   if (ws && sch != schedule::classic)
     prm.graph_maxdeg = ws->maxdeg_of(grph.oR.get_ptr(), n, s);
   else if (sch == schedule::learned)
