@@ -134,6 +134,19 @@ constexpr unsigned long long kSmallWork = 1ull << 18;
 // took 9.4).
 constexpr unsigned long long kTinyWork = 1ull << 16;
 
+// Workgroups of a pull iteration, per compute unit: every workgroup that updates something takes one returning
+// atomic on the queue's counter, 12 ns each on its one line, so 5,376 workgroups
+// need 60 us however little they do.  Settled pulls (BFS, thread per vertex, a
+// few edges per vertex): 3 / 4 / 5 / 7 / 21 per unit take 325 / 320 / 327 / 340 /
+// 383 us for a BFS run on 1M vertices and 16M edges, 446 / 446 / 438 us against
+// 504 on 2M.  Edge-balanced pulls want more workgroups for balance: at most one
+// per kPullWorkPerGroup vertices and edges, at least as many as settled pulls.
+// Widest paths on 200,003 vertices and 3M edges: 2,048 / 2,560 / 3,072 / 4,096 per
+// workgroup take 691 / 612 / 627 / 647 us, on 400,000 865 / 830 / 871 / 977; a
+// graph of 1.6M edges loses 6 % below 800 workgroups, one of 15M 25 % at 1,792.
+constexpr unsigned kPullGroups = 4;
+constexpr unsigned kPullWorkPerGroup = 2560;
+
 // Largest out-degree of the graphs whose tiny push iterations deal whole queue
 // entries to the waves (run_push_few).
 constexpr unsigned kFewDegree = 64;
@@ -306,6 +319,7 @@ struct step_core {
   unsigned collect;     // collect diagnostic counters (work, gathers, active, max degree)
   group_stats* gst;     // kTicketGroups partial slots
   unsigned small_grid;  // least grid of a push iteration (0: push iterations use the whole grid)
+  unsigned pull_grid;   // least grid of a pull iteration (0: pull iterations use the whole grid)
   unsigned* board;      // completion-ticket counters (kTicketWords)
   unsigned max_outdeg;  // largest out-degree of the graph (0: see graph_maxdeg)
   const unsigned* graph_maxdeg;  // device word that holds it, or null
@@ -2215,6 +2229,17 @@ __global__ __launch_bounds__(COMPILE_TIME_DETERMINED_BLOCK_SIZE) void step_kerne
     c.grid = want <= p.small_grid ? p.small_grid
              : want < gridDim.x   ? static_cast<unsigned>(want)
                                   : gridDim.x;
+  }
+  // A pull iteration too runs on fewer workgroups than the launch has (figures
+  // at kPullGroups).
+  if (p.pull_grid && (variant == V_PULL_LB || (variant == V_PULL_T && p.sched.settled_below))) {
+    unsigned long long want = p.pull_grid;
+    if (variant == V_PULL_LB) {
+      unsigned long long const share = (p.nnz + p.m + kPullWorkPerGroup - 1) / kPullWorkPerGroup;
+      // (the source-split pull deals whole rounds of parts)
+      if (share > want) want = (share + kSplitParts - 1) / kSplitParts * kSplitParts;
+    }
+    if (want < gridDim.x) c.grid = static_cast<unsigned>(want);
   }
   bool const idle = blockIdx.x >= c.grid;
   unsigned const wib = threadIdx.x >> 6;

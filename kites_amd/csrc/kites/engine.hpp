@@ -842,6 +842,8 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   prm.board = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(st.ctl) +
                                           offsetof(step_ctl, board));
   prm.small_grid = o.adaptive_grid ? small_grid_of(dev, o) : 0u;
+  prm.pull_grid =
+      o.adaptive_grid ? kPullGroups * static_cast<unsigned>(dev.numComputeUnits()) : 0u;
   unsigned const loop_edges = o.delta && o.persist_edges == detail::kPersistDefaultEdges
                                   ? detail::kPersistFarEdges
                                   : o.persist_edges;
