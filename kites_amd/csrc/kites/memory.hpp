@@ -224,26 +224,32 @@ class device_bitmap : public device_buffer<unsigned long long> {
   std::size_t getnBits() const { return nBits; }
 };
 
-// Several arrays in a few device allocations.  hipMalloc and hipFree of less
-// than 2 MB take 1 us each, larger ones 8 to 125 and 7 to 230 us (a graph and its
-// run state are some twenty arrays): arrays are packed into blocks below that
-// line, and those that reach it share one block.  add() every array, then
-// commit(); the memory is kept, and grown when a later plan needs more.  The
-// arrays do not outlive the arena.
+// Several arrays in a few device allocations.  hipMalloc and hipFree take 1 us
+// each below 2 MB, 8 us up to some 8 MB when a buffer of that size was freed
+// before (up to 125 otherwise), and 55 and 185 us on large sizes; a graph, its
+// build and its run state are some thirty arrays.  Small arrays are packed into
+// blocks below 2 MB, arrays up to kShared have a block of their own, and larger
+// ones share one (allocated last).  Build, first BFS and close of graphs of
+// 210K / 490K / 840K / 1.4M / 2.1M / 16M edges: 1.02 / 1.47 / 2.12 / 2.45 / 2.78
+// / 9.5 ms, with an allocation for each array 1.05 / 1.44 / 2.18 / 3.80 / 4.80 /
+// 14.4; one allocation for all arrays cost a graph of 303K edges 0.3 ms more.
+// add() every array, then commit(); the memory is kept, and grown when a later
+// plan needs more.  The arrays do not outlive the arena.
 class device_arena {
   static constexpr std::size_t kBlock = (std::size_t{2} << 20) - 4096;
+  static constexpr std::size_t kShared = std::size_t{4} << 20;
   struct part {
     std::size_t block, at;
     std::function<void(unsigned char*)> set;
   };
-  std::vector<device_buffer<unsigned char>> mem;   // block 0: the large arrays
+  std::vector<device_buffer<unsigned char>> mem;   // block 0: the arrays that share
   std::vector<std::size_t> need;                   // bytes of every block of the plan
   std::vector<part> parts;
 
   void place(std::size_t count, std::function<void(unsigned char*)> set) {
     count = (count + 255) & ~std::size_t(255);
     std::size_t b = 0;
-    if (count <= kBlock) {
+    if (count < kShared) {
       if (need.size() == 1 || need.back() + count > kBlock) need.push_back(0);
       b = need.size() - 1;
     }
@@ -273,11 +279,13 @@ class device_arena {
   }
   void commit(int dev) {
     if (mem.size() < need.size()) mem.resize(need.size());
-    for (std::size_t b = 0; b < need.size(); ++b)
+    for (std::size_t i = 1; i <= need.size(); ++i) {
+      std::size_t const b = i % need.size();
       if (mem[b].size() < need[b]) {
         mem[b].free();
         mem[b].alloc(need[b], dev);
       }
+    }
     for (auto const& x : parts) x.set(mem[x.block].get_ptr() + x.at);
     parts.clear();
   }
