@@ -8,6 +8,8 @@ with the source tree):
   the host graph generators (gen.cpp) and graph files (graph_files.cpp).
 * ``examples/_build/*``          -- the reference example rewritten against
   the drop-in C++ API, compiled for gfx950.
+* ``tests/native/_build/*``      -- the test programs of the C++ API
+  (tests/native/*.hip), compiled for gfx950.
 
 Run ``python -m kites_amd.build`` (``__graft_entry__.build()`` calls it).
 """
@@ -82,11 +84,13 @@ def build_lib():
     os.replace(tmp, LIB)
 
 
-def build_examples():
-    src_dir = os.path.join(ROOT, "examples")
-    out_dir = os.path.join(src_dir, "_build")
-    os.makedirs(out_dir, exist_ok=True)
-    exes = [os.path.join(out_dir, f[:-4]) for f in sorted(os.listdir(src_dir)) if f.endswith(".hip")]
+def build_programs():
+    exes = []
+    for src_dir in (os.path.join(ROOT, "tests", "native"), os.path.join(ROOT, "examples")):
+        out_dir = os.path.join(src_dir, "_build")
+        os.makedirs(out_dir, exist_ok=True)
+        exes += [os.path.join(out_dir, f[:-4]) for f in sorted(os.listdir(src_dir))
+                 if f.endswith(".hip")]
     _parallel([[hipcc()] + HIP_FLAGS + ["-I", CSRC, e.replace("_build" + os.sep, "") + ".hip",
                                         "-o", e + ".tmp"] for e in exes])
     for e in exes:
@@ -95,7 +99,7 @@ def build_examples():
 
 def build():
     build_lib()
-    build_examples()
+    build_programs()
 
 
 if __name__ == "__main__":

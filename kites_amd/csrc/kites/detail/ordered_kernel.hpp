@@ -72,6 +72,11 @@ struct ordered_shape {
   static constexpr unsigned rows = slots / 64;
   static constexpr unsigned batch = small ? 4 : 2;          // rows of 64 edges in flight per wave
   static constexpr unsigned heavy_unroll = small ? 2 : 1;   // heavy chunks in flight per wave
+  // A row's segment heads (4 bytes an edge) may lie where its partials will: a
+  // batch of rows reads its heads before it writes its partials.  Partials of
+  // more than 4 bytes would reach into the heads of later batches, which then
+  // have an area of their own.
+  static constexpr bool heads_apart = sizeof(vT) > sizeof(unsigned);
   static_assert(rows % batch == 0, "whole batches of rows");
 };
 
@@ -403,9 +408,10 @@ void ordered_kernel(P p) {
   constexpr unsigned kW = S::waves;
   constexpr unsigned kRows = S::rows, kB = S::batch;
   // A wave's partials; before a row's partials are written, its words hold the
-  // row's segment heads.
+  // row's segment heads (ordered_shape::heads_apart: an array of their own).
   constexpr unsigned kSlotBytes = S::slots * (sizeof(vT) < 4 ? 4 : sizeof(vT));
   __shared__ __align__(16) unsigned char slot_s[kW][(kSlotBytes + 15) / 16 * 16];
+  __shared__ unsigned head_s[kW][S::heads_apart ? S::slots : 1];
   __shared__ vT acc_s[kW][64];
   __shared__ unsigned long long words_s[kW][64];
   __shared__ unsigned excl_s[kW][64], base_s[kW][64];
@@ -423,7 +429,8 @@ void ordered_kernel(P p) {
   unsigned long long* const out = p.bm + static_cast<unsigned long long>((iter + 1) & 1) * p.nwords;
   unsigned const t = threadIdx.x, lane = lane_id(), wib = readfirstlane(t >> 6);
   vT* const slot = reinterpret_cast<vT*>(slot_s[wib]);
-  unsigned* const head = reinterpret_cast<unsigned*>(slot_s[wib]);
+  unsigned* const head =
+      S::heads_apart ? head_s[wib] : reinterpret_cast<unsigned*>(slot_s[wib]);
   vT* const acc = acc_s[wib];
   unsigned* const act = act_s[wib];
   ordered_wave ow;
@@ -557,7 +564,7 @@ void ordered_kernel(P p) {
         src[u] = p.C[e[u]];
         w[u] = p.E[e[u]];
       }
-      wave_lds_sync();   // the heads are read; their words take the partials
+      wave_lds_sync();   // the heads are read; their words may take the partials
 #pragma unroll
       for (unsigned u = 0; u < kB; ++u) x[u] = Vin[src[u]];
       if (by_source) {
