@@ -20,8 +20,8 @@
 // source vertex, two lists that take turns): a thread needs no search to find
 // its edges.  An iteration is three accesses long:
 //   1. the edge's destination and weight and V[source];
-//   2. V[destination]; then a barrier, so that every thread has read the values
-//      the iteration starts from;
+//   2. V[destination], waited for; then a barrier, so that every thread has read
+//      the values the iteration starts from;
 //   3. for a candidate below that value, one returning atomic min, and beside it
 //      the destination's out-offsets.  The thread whose atomic returns the
 //      starting value lowered the vertex first and appends it (no other does, so
@@ -30,10 +30,11 @@
 // The decision of the next iteration is made by every thread from the totals in
 // LDS (three sets of counters take turns), so the iteration has two barriers.
 // Microseconds per iteration (BFS on grids of 16 / 64 / 256 / 480 columns, the
-// queue two thirds of that): 1.9 / 2.1 / 3.4 / 6.0; a form that staged the queue
+// queue two thirds of that): 1.9 / 2.1 / 3.6 / 6.1 (without the wait in front of
+// the barrier 1.9 / 2.1 / 3.4 / 6.0); a form that staged the queue
 // in LDS, searched each edge's entry and claimed bits took 4.3 / 4.6 / 6.0 /
-// 9.2; step_kernel takes 6.2 / 6.5 / 6.9 / 7.0.  Near-far SSSP: 2.8 / 3.0 /
-// 6.1 / 8.5 against 5.9 / 6.4 / 11.1 / 11.9, step_kernel 8.9 / 9.5 / 10.0 /
+// 9.2; step_kernel takes 6.2 / 6.5 / 6.9 / 7.0.  Near-far SSSP: 2.7 / 3.0 /
+// 5.9 / 8.3 against 5.9 / 6.4 / 11.1 / 11.9, step_kernel 8.9 / 9.5 / 10.0 /
 // 10.0.  The slope, 2.3 ns per edge, is the unit's scattered accesses, so
 // BFS queues of more than about 2,048 out-edges go to step_kernel: at 4,096
 // grids of 700 to 2,000 columns take 7.5 to 9.4.
@@ -237,6 +238,10 @@ __device__ __forceinline__ void persist_push(P& p, persist_smem<vT>& sm, unsigne
   for (unsigned k = 0; k < R; ++k) cand[k] = edge_value(p.fn, sm.slot[t], val[k], &w[k]);
 #pragma unroll
   for (unsigned k = 0; k < R; ++k) ok[k] = ok[k] && cand[k] < start[k];
+  // (the barrier alone waits for no load: one still in flight could read what
+  // another wave's atomic has written, and two threads would then take theirs
+  // for the first relaxation of a vertex and append it twice)
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   vT old[R];
   unsigned b[R], deg[R];
