@@ -14,6 +14,7 @@ namespace {
 
 using kites_capi::kInf;
 using kites_capi::need;
+using kites_capi::run_from_start;
 using kites_capi::settle_bfs;
 using kites_capi::to_options;
 using kites_capi::with_functors;
@@ -70,8 +71,9 @@ namespace kites_capi {
 
 // The reference protocol's frontier of a start recorded by kites_graph_init or
 // kites_graph_init_sources: the sources' out-neighbours (every vertex for
-// min-label CC is marked with the values).  Only the reference algorithm reads
-// it; delta schedules start from the recorded sources themselves.
+// min-label CC is marked with the values).  The reference algorithm reads it,
+// and a run that finds no recorded start (run_from_start); delta schedules
+// start from the recorded sources themselves.
 void mark_start(kites_graph* g) {
   auto& dg = *g->g;
   g->dev->setAsActive();
@@ -496,12 +498,11 @@ int kites_graph_run(kites_graph* g, int32_t algo, const kites_run_opts* o, kites
   kites::options opt = to_options(g, o);
   opt.report = &rep;
   settle_bfs(g, algo, opt);
-  if (opt.sched == kites::schedule::classic) kites_capi::mark_start(g);
   // The recorded start is consumed by this run, as the frontier is.
-  g->seed = kites::options::seeding::none;
-  g->unit_start = false;
-  with_functors(algo, [&](auto fi, auto fn, auto fr, auto fu) {
-    kites::process<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt);
+  run_from_start(g, rep, opt.sched == kites::schedule::classic, [&] {
+    with_functors(algo, [&](auto fi, auto fn, auto fr, auto fu) {
+      kites::process<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt);
+    });
   });
   if (opt.keep_stats) g->stats = rep.stats;
   if (info) {
@@ -572,11 +573,13 @@ int kites_graph_record(kites_graph* g, int32_t algo, const kites_run_opts* o,
   need(opt.sched != kites::schedule::classic, "the recorder needs a delta schedule");
   opt.record = &rec;
   opt.record_rollout = rollout_variant;
+  kites::run_report rep;
+  opt.report = &rep;
   settle_bfs(g, algo, opt);
-  g->seed = kites::options::seeding::none;
-  g->unit_start = false;
-  with_functors(algo, [&](auto fi, auto fn, auto fr, auto fu) {
-    kites::process<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt);
+  run_from_start(g, rep, false, [&] {
+    with_functors(algo, [&](auto fi, auto fn, auto fr, auto fu) {
+      kites::process<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt);
+    });
   });
   if (count) *count = static_cast<uint32_t>(rec.size());
   if (out) std::memcpy(out, rec.data(), std::min<std::size_t>(cap, rec.size()) * sizeof(kites_variant_sample));

@@ -71,6 +71,32 @@ inline int fail(std::exception const& e) {
 
 void mark_start(kites_graph* g);   // capi.hip
 
+// Runs `run`, which fills `rep`, on the start recorded by kites_graph_init or
+// kites_graph_init_sources.  The start is recorded for one run; a call that
+// failed before it took the start over leaves the start's frontier in its
+// place, from which the next run of any schedule begins.
+template <class Run>
+void run_from_start(kites_graph* g, kites::run_report const& rep, bool classic, Run&& run) {
+  if (classic) mark_start(g);
+  auto const seed = g->seed;
+  g->seed = kites::options::seeding::none;
+  g->unit_start = false;
+  try {
+    run();
+  } catch (...) {
+    if (!rep.started) {
+      g->seed = seed;
+      try {
+        mark_start(g);
+      } catch (...) {
+        // (an error that is already being reported)
+      }
+      g->seed = kites::options::seeding::none;
+    }
+    throw;
+  }
+}
+
 inline void need(bool c, const char* what) {
   if (!c) throw std::invalid_argument(what);
 }

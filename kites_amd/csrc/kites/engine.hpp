@@ -68,6 +68,9 @@ struct variant_sample {
 
 // Per-run report (optional output of process()).
 struct run_report {
+  // The run took the start over: the values and the initial frontier are its
+  // own from then on.  A call that failed before left both as they were.
+  bool started = false;
   unsigned iterations = 0;
   double ms = 0.0;             // device time of the iteration loop (hipEvents)
   bool delta = false;          // delta variants were allowed
@@ -603,6 +606,7 @@ void run_ordered(ordered_view<vT, eT> const& g, gpu& dev, stream& s, ordered_wor
   using S = ordered_shape<vT>;
   using P = ordered_params<vT, eT, FI, FN, FR, FU>;
   std::size_t const n = g.n, m = g.m;
+  if (o.report) o.report->started = true;   // (its caller clears the frontier, also on failure)
   unsigned const nwords = static_cast<unsigned>((n + 63) / 64 + 1);
   unsigned const ntasks = static_cast<unsigned>(m / S::task_edges + 1);
   // a heavy vertex holds more than S::light in-edges
@@ -886,6 +890,7 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
     hipLaunchKernelGGL(list, dim3(1), dim3(COMPILE_TIME_DETERMINED_BLOCK_SIZE), 0, s.get(), kp,
                        o.seed_list, o.seed_count);
   }
+  if (o.report) o.report->started = true;
   KITES_HIP_CHECK(hipPeekAtLastError());
   // (a bitmap longer than the run's slots: vertex groups finer than 64 ids)
   if (grph.vBitmapEven.sizeInBytes() > fb)
@@ -974,6 +979,7 @@ template <launch launchMode, class vT, class eT, class vIdxT, class funcInitT,
 void process(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcInit,
              funcCompNbrT funcCompNbr, funcRedT funcRed, funcUpdT funcUpd, options const& o) {
   using namespace detail;
+  if (o.report) o.report->started = false;
   dev.setAsActive();
   std::size_t const n = grph.get_num_vertices();
   if (o.verbose) {
@@ -1002,6 +1008,7 @@ template <launch launchMode, class vT, class eT, class vIdxT, class funcInitT,
 void process_noalloc(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcInit,
                      funcCompNbrT funcCompNbr, funcRedT funcRed, funcUpdT funcUpd,
                      options const& o, detail::run_state& st) {
+  if (o.report) o.report->started = false;
   if (o.keep_stats || o.verbose)
     throw std::invalid_argument("kites::process_noalloc: statistics and verbose output allocate");
   std::size_t const n = grph.get_num_vertices();

@@ -94,9 +94,6 @@ int kites_sssp_u32_noalloc(kites_graph* g, uint32_t source, const kites_run_opts
   int rc = kites_graph_init(g, KITES_ALGO_SSSP, source);
   if (rc) return rc;
   kites::options opt = kites_capi::to_options(g, o);
-  if (opt.sched == kites::schedule::classic) kites_capi::mark_start(g);
-  g->seed = kites::options::seeding::none;   // the recorded start is consumed
-
   kites::detail::run_state st;
   st.bm = reinterpret_cast<unsigned long long*>(base + kOffBm);
   st.q = reinterpret_cast<unsigned*>(base + kOffQ);
@@ -112,8 +109,10 @@ int kites_sssp_u32_noalloc(kites_graph* g, uint32_t source, const kites_run_opts
 
   kites::run_report rep;
   opt.report = &rep;
-  kites_capi::with_sssp([&](auto fi, auto fn, auto fr, auto fu) {
-    kites::process_noalloc<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt, st);
+  kites_capi::run_from_start(g, rep, opt.sched == kites::schedule::classic, [&] {
+    kites_capi::with_sssp([&](auto fi, auto fn, auto fr, auto fu) {
+      kites::process_noalloc<kites::launch::sync>(*g->g, *g->dev, fi, fn, fr, fu, opt, st);
+    });
   });
   if (info) {
     info->iterations = rep.iterations;
