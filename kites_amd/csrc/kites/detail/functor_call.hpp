@@ -88,12 +88,14 @@ __host__ __device__ __forceinline__ bool update_at(FU& fu, vT& slot, vT old) {
 }
 
 // nv = redF(old, cand); returns updF(nv, old).  `work` and `slot`: LDS slots of
-// the lane, `slot` holding `cand`.
+// the lane (edge_value leaves `cand` in no slot when nbrCompF takes plain
+// references, so a volatile redF gets it put there).
 template <class FR, class FU, class vT>
 __host__ __device__ __forceinline__ bool combine(FR& fr, FU& fu, vT old, vT cand, vT& work, vT& slot,
                                         vT& nv) {
   if constexpr (std::is_invocable<FR&, volatile vT&, volatile vT&>::value) {
     as_volatile(work) = old;
+    as_volatile(slot) = cand;
     fr(as_volatile(work), as_volatile(slot));
     bool const u = update_at(fu, work, old);
     nv = as_volatile(work);

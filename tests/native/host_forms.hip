@@ -1,4 +1,5 @@
 // host_forms.hip -- checks of the engine's headers that need no GPU.
+#include "forms.hpp"
 #include "native.hpp"
 
 using namespace native;
@@ -27,9 +28,59 @@ void ordered_layout() {
   report("ordered segment heads of " + std::to_string(BYTES) + "-byte values", bad == 0);
 }
 
+// The four functors of a max-min set, each in either form, through the helpers
+// the kernels call them with.  The slots hold what an earlier edge left.
+template <bool I, bool N, bool R, bool U>
+void functor_mix() {
+  using namespace kites::detail;
+  using vT = int;
+  copy_init<I, vT> fi;
+  narrow<N, vT, unsigned> fn;
+  take_max<R, vT> fr;
+  more<U, vT> fu;
+  bool ok = true;
+  for (vT old : {0, 3, 7, 9})
+    for (vT src : {0, 2, 7, 100})
+      for (unsigned w : {1u, 7u, 50u})
+        for (vT left : {-1, 0, 8, 1000}) {
+          vT const cand = src < static_cast<vT>(w) ? src : static_cast<vT>(w);
+          vT const want = old < cand ? cand : old;
+          unsigned e = w;
+          vT slot = left, work = left, nv = left;
+          ok = ok && edge_value(fn, slot, src, &e) == cand;
+          // a push: the partial as returned, the slots as edge_value left them
+          slot = N ? cand : left;
+          bool const moved = combine(fr, fu, old, cand, work, slot, nv);
+          ok = ok && moved == (want > old) && (!moved || nv == want);
+          // a pull: slots in place
+          vT acc = left, part = left;
+          init_at(fi, acc, old);
+          edge_value_at(fn, part, src, &e);
+          reduce_at(fr, acc, part);
+          ok = ok && part == cand && acc == want && update_at(fu, acc, old) == (want > old);
+        }
+  std::string const names = std::string("functor forms ") + (I ? "v" : "p") + (N ? "v" : "p") +
+                            (R ? "v" : "p") + (U ? "v" : "p");
+  report(names, ok);
+}
+
+template <bool I, bool N, bool R>
+void functor_mixes() {
+  functor_mix<I, N, R, false>();
+  functor_mix<I, N, R, true>();
+}
+
 }  // namespace
 
 int main() {
+  functor_mixes<false, false, false>();
+  functor_mixes<false, false, true>();
+  functor_mixes<false, true, false>();
+  functor_mixes<false, true, true>();
+  functor_mixes<true, false, false>();
+  functor_mixes<true, false, true>();
+  functor_mixes<true, true, false>();
+  functor_mixes<true, true, true>();
   ordered_layout<1>();
   ordered_layout<2>();
   ordered_layout<4>();

@@ -30,3 +30,9 @@ def test_headers_on_the_host():
 def test_ordered_value_types():
     out = _run("ordered_types")
     assert out.count("ok:") == 12
+
+
+@pytest.mark.gpu
+def test_functor_forms():
+    out = _run("functor_forms")
+    assert out.count("ok:") == 8 * 2 * 21
