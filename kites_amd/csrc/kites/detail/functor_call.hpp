@@ -25,6 +25,18 @@ __host__ __device__ __forceinline__ volatile T& as_volatile(T& x) {
   return *reinterpret_cast<volatile T*>(&x);
 }
 
+// nbrCompF takes the edge as a pointer to const: it can only read it, so a
+// kernel may call it for an edge whose partial is then dropped.  (One that takes
+// the reference's eT* may write through it: each call then stands for one walk
+// of that edge.)  Either way the pointer is the edge's place in the graph's array.
+template <class FN, class vT, class eT>
+constexpr bool reads_edge = std::is_invocable<FN&, volatile vT&, vT, const eT*>::value ||
+                            std::is_invocable<FN&, vT&, vT, const eT*>::value;
+
+// nbrCompF works on its lane's LDS slot (volatile references).
+template <class FN, class vT, class eT>
+constexpr bool takes_slot = std::is_invocable<FN&, volatile vT&, vT, eT*>::value;
+
 // nbrCompF(partial, srcV, edge); `slot`: an LDS slot of the calling lane.
 template <class FN, class vT, class eT>
 __host__ __device__ __forceinline__ vT edge_value(FN& fn, vT& slot, vT src, eT* edge) {

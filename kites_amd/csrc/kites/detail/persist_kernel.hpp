@@ -220,22 +220,31 @@ __device__ __forceinline__ void persist_push(P& p, persist_smem<vT>& sm, unsigne
   unsigned const t = threadIdx.x;
   unsigned idx[R], dst[R];
   vT val[R], cand[R], start[R];
-  eT w[R];
   bool ok[R];
-  // (a thread without an edge repeats the list's first one, and drops it)
+  // A thread without an edge repeats the list's first one and drops it; the
+  // functor is called for it only if it cannot write the edge.  Functors in
+  // registers are called among the loads (behind all of them near-far
+  // iterations of 16 columns take 2.82 us instead of 2.76), functors in LDS
+  // slots, whose flat accesses wait for every load, after them.
+  constexpr bool kRead = reads_edge<decltype(p.fn), vT, eT>;
+  constexpr bool kEarly = kRead && !takes_slot<decltype(p.fn), vT, eT>;
 #pragma unroll
   for (unsigned k = 0; k < R; ++k) {
     unsigned const e = t + k * kPersistBlock;
     ok[k] = e < E;
     idx[k] = sm.idx[cur][ok[k] ? e : 0u];
-    val[k] = load_agent(p.V + sm.src[cur][ok[k] ? e : 0u]);
     dst[k] = p.oC[idx[k]];
-    w[k] = p.oE[idx[k]];
+    val[k] = load_agent(p.V + sm.src[cur][ok[k] ? e : 0u]);
+    cand[k] = vT{};
+    if constexpr (kEarly) cand[k] = edge_value(p.fn, sm.slot[t], val[k], p.oE + idx[k]);
+  }
+  if constexpr (!kEarly) {
+#pragma unroll
+    for (unsigned k = 0; k < R; ++k)
+      if (kRead || ok[k]) cand[k] = edge_value(p.fn, sm.slot[t], val[k], p.oE + idx[k]);
   }
 #pragma unroll
   for (unsigned k = 0; k < R; ++k) start[k] = load_agent(p.V + dst[k]);
-#pragma unroll
-  for (unsigned k = 0; k < R; ++k) cand[k] = edge_value(p.fn, sm.slot[t], val[k], &w[k]);
 #pragma unroll
   for (unsigned k = 0; k < R; ++k) ok[k] = ok[k] && cand[k] < start[k];
   // (the barrier alone waits for no load: one still in flight could read what

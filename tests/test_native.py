@@ -36,3 +36,9 @@ def test_ordered_value_types():
 def test_functor_forms():
     out = _run("functor_forms")
     assert out.count("ok:") == 8 * 2 * 21
+
+
+@pytest.mark.gpu
+def test_edge_pointer():
+    out = _run("edge_pointer")
+    assert out.count("ok:") == 10
