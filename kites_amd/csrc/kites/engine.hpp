@@ -595,7 +595,8 @@ struct ordered_view {
 };
 
 // The ordered mode's loop over the view `g` (detail/ordered_kernel.hpp): two
-// launches per iteration, the iteration index, the activity form and the done
+// launches per iteration (three for a functor that may write the edge), the
+// iteration index, the activity form and the done
 // flag on the device; the host queues kOrderedChunk iterations and then reads
 // the control header once.
 constexpr unsigned kOrderedChunk = 4;
@@ -629,6 +630,8 @@ void run_ordered(ordered_view<vT, eT> const& g, gpu& dev, stream& s, ordered_wor
   ws.mem.begin();
   ws.mem.add(prm.W, n);
   ws.mem.add(prm.bm, 2 * static_cast<std::size_t>(nwords));
+  constexpr bool kRead = reads_edge<FN, vT, eT>;
+  ws.mem.add(prm.abm, kRead ? 0 : nwords);
   ws.mem.add(prm.hasin, nwords);
   ws.mem.add(prm.tstart, static_cast<std::size_t>(ntasks) + 1);
   ws.mem.add(prm.hv, hcap);
@@ -666,6 +669,10 @@ void run_ordered(ordered_view<vT, eT> const& g, gpu& dev, stream& s, ordered_wor
   unsigned long long launched = 0;
   for (;;) {
     for (unsigned k = 0; k < kOrderedChunk; ++k) {
+      if constexpr (!kRead) {
+        auto const activate = &ordered_activate_kernel<P>;
+        hipLaunchKernelGGL(activate, dim3(blocks(nwords, 4)), dim3(256), 0, s.get(), prm);
+      }
       hipLaunchKernelGGL(heavy, dim3(hgrid), dim3(S::block), 0, s.get(), prm);
       hipLaunchKernelGGL(kern, dim3(mgrid), dim3(S::block), 0, s.get(), prm);
     }

@@ -78,7 +78,7 @@ int kites_pagerank_f32(kites_graph* g, float damping, float tol, uint32_t max_it
   // product and a sum each round on their own, as the combine order defines.
   float const base = 1.0f - damping;
   auto initF = [base] __host__ __device__(float& locV, float&) { locV = base; };
-  auto nbrF = [damping] __host__ __device__(float& partialV, float srcV, float* connE) {
+  auto nbrF = [damping] __host__ __device__(float& partialV, float srcV, const float* connE) {
 #pragma clang fp contract(off)
     partialV = damping * srcV * (*connE);
   };

@@ -1,10 +1,12 @@
 // ordered_types.hip -- options::ordered on value types of 4 to 32 bytes, bit
-// for bit against the combine order's definition run on the host.
+// for bit against the combine order's definition run on the host, and the calls
+// of a functor that writes its edges.
 //
 // The graph has no cycles (every source id is below its destination's), so any
 // functor set settles; in-lists of 1 to 64 edges lie side by side, so that a
 // task's window holds more than 256 light in-edges, with lists at both sides of
 // the light limit (64) and of a window (448) between them.
+#include "forms.hpp"
 #include "native.hpp"
 
 using namespace native;
@@ -154,6 +156,68 @@ void run(csr const& g, kites::gpu& dev, const char* name) {
   }
 }
 
+// A functor that writes the edge counts its calls there: once per iteration and
+// in-edge of the active vertices, as the definition has it.
+struct counted {
+  unsigned w, calls;
+};
+template <bool VOL, class vT>
+struct counting {
+  __host__ __device__ void operator()(ref<VOL, vT> part, vT src, counted* e) const {
+    e->calls += 1;
+    part = scale(src, e->w);
+  }
+};
+template <bool VOL, class vT>
+struct sum {
+  __host__ __device__ void operator()(ref<VOL, vT> l, ref<VOL, vT> r) const {
+    vT const a = l, b = r;
+    l = fold(a, b);
+  }
+};
+template <bool VOL, class vT>
+struct seven {
+  __host__ __device__ void operator()(ref<VOL, vT> loc, vT&) const { loc = make<vT>(7); }
+};
+template <bool VOL, class vT>
+struct moves {
+  __host__ __device__ bool operator()(ref<VOL, vT> nv, vT old) const {
+    vT const x = nv;
+    return !(x == old);
+  }
+};
+
+template <bool VOL, class vT>
+void calls(csr const& g, kites::gpu& dev, const char* name) {
+  std::vector<counted> E(g.m());
+  numbers rnd(12);
+  for (counted& e : E) e = counted{1 + rnd.below(9), 0};
+  std::vector<vT> V0(g.n);
+  for (unsigned v = 0; v < g.n; ++v) V0[v] = make<vT>(v + 1);
+  for (unsigned some : {0u, 1u}) {
+    std::vector<char> active(g.n, 1);
+    if (some)
+      for (unsigned v = 0; v < g.n; ++v) active[v] = v % 9 == 4;
+    std::string const what = std::string("ordered calls, ") + name + (VOL ? ", volatile" : ", plain") +
+                             (some ? ", some active" : ", all active");
+    announce(what);
+    std::vector<vT> exp = V0;
+    std::vector<counted> e2 = E;
+    unsigned const it = reference(g, e2, exp, active, seven<VOL, vT>{}, counting<VOL, vT>{},
+                                  sum<VOL, vT>{}, moves<VOL, vT>{});
+    auto d = upload<vT, counted>(g, E, dev);
+    start(*d, V0, active);
+    kites::run_report rep;
+    kites::options o;
+    o.ordered = true;
+    o.report = &rep;
+    kites::process<kites::launch::sync>(*d, dev, seven<VOL, vT>{}, counting<VOL, vT>{},
+                                        sum<VOL, vT>{}, moves<VOL, vT>{}, o);
+    report(what, rep.iterations == it && same(to_host(d->V.get_ptr(), g.n), exp) &&
+                     same(to_host(d->E.get_ptr(), g.m()), e2));
+  }
+}
+
 }  // namespace
 
 int main() {
@@ -165,5 +229,9 @@ int main() {
   run<mixed<12>>(g, dev, "12-byte struct");
   run<mixed<16>>(g, dev, "16-byte struct");
   run<mixed<32>>(g, dev, "32-byte struct");
+  calls<false, float>(g, dev, "float");
+  calls<true, float>(g, dev, "float");
+  calls<false, long long>(g, dev, "long long");
+  calls<true, long long>(g, dev, "long long");
   return finish();
 }

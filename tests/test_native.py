@@ -29,7 +29,7 @@ def test_headers_on_the_host():
 @pytest.mark.gpu
 def test_ordered_value_types():
     out = _run("ordered_types")
-    assert out.count("ok:") == 12
+    assert out.count("ok:") == 20
 
 
 @pytest.mark.gpu
