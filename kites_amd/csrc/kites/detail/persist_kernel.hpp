@@ -88,6 +88,8 @@ constexpr unsigned kPersistEdges = kPersistBlock * kPersistRounds;
 // 6.0 / 8.4 / 8.8 / 8.5 / 8.5 with 4,096.
 constexpr unsigned kPersistDefaultEdges = 2048;
 constexpr unsigned kPersistFarEdges = 4096;
+// options::persist_edges left alone: one of the two (no limit a caller sets).
+constexpr unsigned kPersistAutoEdges = 0xFFFFFFFEu;
 // Out-lists up to this long are written to the edge list by the lane that
 // appends the vertex, longer ones by its wave.
 constexpr unsigned kPersistLane = 16;

@@ -115,10 +115,10 @@ struct options {
   // one-workgroup loop that runs every iteration whose queue fits it
   // (detail/persist_kernel.hpp) in one launch.  Needs adaptive_grid.
   // persist_edges: the largest out-edge total of a queue the loop takes (at most
-  // detail::kPersistEdges; left at the default, near-far runs take
-  // detail::kPersistFarEdges).
+  // detail::kPersistEdges; left at the default detail::kPersistDefaultEdges,
+  // near-far runs detail::kPersistFarEdges).
   bool persist = true;
-  unsigned persist_edges = detail::kPersistDefaultEdges;
+  unsigned persist_edges = detail::kPersistAutoEdges;
   // Edge-balanced pull over the source-split in-CSR (split.hpp): each XCD
   // gathers source values from its own eighth of V.  Holds one more copy of
   // C and E, built on the first run that sets it (delta schedules only).
@@ -855,9 +855,9 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   prm.small_grid = o.adaptive_grid ? small_grid_of(dev, o) : 0u;
   prm.pull_grid =
       o.adaptive_grid ? kPullGroups * static_cast<unsigned>(dev.numComputeUnits()) : 0u;
-  unsigned const loop_edges = o.delta && o.persist_edges == detail::kPersistDefaultEdges
-                                  ? detail::kPersistFarEdges
-                                  : o.persist_edges;
+  unsigned const loop_edges = o.persist_edges != detail::kPersistAutoEdges ? o.persist_edges
+                              : o.delta                                    ? detail::kPersistFarEdges
+                                        : detail::kPersistDefaultEdges;
   prm.persist_edges = o.persist ? std::min(loop_edges, detail::kPersistEdges) : 0u;
   if (ws && sch != schedule::classic)
     prm.graph_maxdeg = ws->maxdeg_of(grph.oR.get_ptr(), n, s);

@@ -46,3 +46,22 @@ def test_a_vertex_enters_a_queue_once(w):
         assert np.array_equal(got, want)
         assert max(x["count"] for x in d.stats()) <= d.n
     d.close()
+
+
+@pytest.mark.parametrize("persist", [True, 2047, 2048, 2049, 3024, 3025, 4096, 16384])
+@pytest.mark.parametrize("delta", [0, 1 << 20])
+def test_out_edge_limit_is_the_one_asked_for(persist, delta):
+    """Queues of 55 x 55 = 3,025 out-edges: the loop runs them when the limit
+    reaches that far.  Left at the default, plain runs stop at 2,048 and
+    near-far runs at 4,096; 2,048 asked for is 2,048 in both."""
+    h, src = _layers(55, 60, 1)
+    d = K.DeviceGraph(h)
+    case(f"loop limit {persist} delta {delta}")
+    limit = (4096 if delta else 2048) if persist is True else min(int(persist), 4096)
+    got, _ = d.solve("sssp", src, persist=persist, delta=delta, keep_stats=True)
+    R, C, E, *_ = h.arrays()
+    assert np.array_equal(got, O.dijkstra(R, C, E, src))
+    st = d.stats()
+    full = [b["variant"] == 11 for a, b in zip(st[20:], st[21:]) if a["sum_outdeg"] == 3025]
+    assert len(full) >= 30 and all(f == (3025 <= limit) for f in full)
+    d.close()
