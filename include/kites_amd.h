@@ -72,7 +72,8 @@ typedef struct kites_run_opts {
   int32_t use_graph;        /* replay iteration chunks from a captured hipGraph */
   int32_t chunk;            /* iterations per chunk (tiny frontiers and small graphs; others
                                are launched one at a time, a few ahead) */
-  int32_t grid;             /* workgroups per launch, 0 = occupancy-derived */
+  int32_t grid;             /* workgroups per launch; 0, or at least three rounds of the
+                               resident ones: the engine's choice for the graph's size */
   uint32_t max_iterations;
   int32_t keep_stats;       /* keep per-iteration statistics (kites_graph_stats) */
   float margin;             /* learned: keep the plain choice unless another variant is

@@ -102,7 +102,8 @@ struct options {
   unsigned max_iterations = 1u << 16;
   bool use_graph = true;
   unsigned chunk = 16;
-  unsigned grid = 0;                     // 0 = occupancy-derived
+  unsigned grid = 0;                     // workgroups of a launch; 0 = three rounds of the
+                                         // resident ones, small graphs fewer (run_loop)
   bool adaptive_grid = true;             // small grid for chunks of small push frontiers
   unsigned small_grid = 0;               // workgroups of that grid (0 = one per compute unit)
   unsigned tiny_grid = 0;                // after a tiny push frontier (0 = a quarter of those)
@@ -330,14 +331,20 @@ unsigned run_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options cons
   auto kern = &step_kernel<DELTA, MIN_FAST, NF, P>;
   unsigned const chunk = std::max(1u, o.chunk);
   bool const follow = prm.progress && o.pipeline;
+  // A grid that was asked for is taken literally below the resident workgroups'
+  // three rounds; from there on it asks for the whole chip, as 0 does, and the
+  // graph's size decides (SSSP on R-MAT graphs of 2^9 / 2^12 / 2^14 vertices with
+  // 21 workgroups per CU: 151 / 246 / 266 us literally, 129 / 186 / 213 so).
+  bool const whole = o.adaptive_grid &&
+                     (!o.grid || grid >= step_grid<DELTA, MIN_FAST, NF, P>(dev, 0));
   bool const small_graph =
-      DELTA && o.adaptive_grid && !o.grid &&
+      DELTA && whole &&
       static_cast<unsigned long long>(prm.n) + prm.m <= kSmallWork;
   unsigned g[3];
   g[1] = std::min(grid, small_grid_of(dev, o));
   g[2] = std::min(g[1], tiny_grid_of(dev, o));
   g[0] = grid;
-  if (o.adaptive_grid && !o.grid) {
+  if (whole) {
     unsigned long long const want =
         (static_cast<unsigned long long>(prm.n) + prm.m + kWorkPerGroup - 1) / kWorkPerGroup;
     if (want < grid) g[0] = std::max(g[1], static_cast<unsigned>(want));
