@@ -219,12 +219,17 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
     for (std::size_t l = issued.load();
          l < launches && (l < 2 || moved[l - 2].load() == chunks_of(l - 2)); ++l) {
       std::size_t const at = l * half, count = std::min(half, bytes - at);
-      hipLaunchKernelGGL(copy_out_kernel, dim3(kCopyGrid), dim3(256), 0, s, rows, stride, K,
-                         static_cast<unsigned long long>(at / sizeof(unsigned)),
-                         static_cast<unsigned>(count / sizeof(unsigned)),
-                         reinterpret_cast<unsigned*>(ring->half(l)), ring->flags(l),
-                         number + static_cast<unsigned>(l));
-      hipError_t const e = hipGetLastError();
+      unsigned long long first = at / sizeof(unsigned);
+      unsigned values = static_cast<unsigned>(count / sizeof(unsigned));
+      unsigned* to = reinterpret_cast<unsigned*>(ring->half(l));
+      unsigned* flags = ring->flags(l);
+      unsigned mark = number + static_cast<unsigned>(l), step = stride, columns = K;
+      const unsigned* from = rows;
+      void* args[] = {&from, &step, &columns, &first, &values, &to, &flags, &mark};
+      // (this launch's own status: the thread's last error may be an earlier
+      // call's, which was reported there)
+      hipError_t const e = hipLaunchKernel(reinterpret_cast<const void*>(&copy_out_kernel),
+                                           dim3(kCopyGrid), dim3(256), args, 0, s);
       if (e != hipSuccess) error.store(static_cast<int>(e));
       issued.store(l + 1);
     }
