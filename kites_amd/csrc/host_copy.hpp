@@ -28,6 +28,9 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
+#include <fstream>
+#include <istream>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -167,14 +170,35 @@ static __global__ __launch_bounds__(256) void copy_out_kernel(const unsigned* __
   }
 }
 
-// Threads for a copy: one per megabyte (a helper takes about 20 us to start).
+// Whole CPUs of a control group's CPU time (quota microseconds per period): at
+// least one, all when there is no limit ("max", or a negative quota).
+inline std::size_t quota_cpus(std::istream& quota, std::istream& period) {
+  long long q = 0, p = 0;
+  if (!(quota >> q) || !(period >> p) || q <= 0 || p <= 0)
+    return std::numeric_limits<std::size_t>::max();
+  return static_cast<std::size_t>(std::max(1ll, q / p));
+}
+
+// The limit of the container the process runs in (read once: 40 us).
+inline std::size_t container_cpus() {
+  static std::size_t const cpus = [] {
+    std::ifstream both("/sys/fs/cgroup/cpu.max");
+    if (both) return quota_cpus(both, both);
+    std::ifstream q("/sys/fs/cgroup/cpu/cpu.cfs_quota_us"), p("/sys/fs/cgroup/cpu/cpu.cfs_period_us");
+    return quota_cpus(q, p);
+  }();
+  return cpus;
+}
+
+// Threads for a copy: one per megabyte (a helper takes about 20 us to start), as
+// many as the process may run at once.
 inline unsigned copy_threads(std::size_t bytes) {
   cpu_set_t set;
   std::size_t cpus = 1;
   if (sched_getaffinity(0, sizeof(set), &set) == 0)
     cpus = static_cast<std::size_t>(std::max(1, CPU_COUNT(&set)));
-  return static_cast<unsigned>(
-      std::max<std::size_t>(1, std::min<std::size_t>({kCopyThreads, cpus, bytes >> 20})));
+  return static_cast<unsigned>(std::max<std::size_t>(
+      1, std::min<std::size_t>({kCopyThreads, cpus, container_cpus(), bytes >> 20})));
 }
 
 // n x K values (row-major) from device rows `stride` values apart (16-byte
@@ -247,7 +271,7 @@ inline void copy_columns(unsigned* dst, const unsigned* rows, std::size_t n, uns
         auto since = std::chrono::steady_clock::now();
         while (__atomic_load_n(flag + b, __ATOMIC_ACQUIRE) != number + l) {
           if (error.load()) return;
-          __builtin_ia32_pause();
+          kites::detail::wait_turn(spins);
           // A stream that has failed, or has been idle for seconds, raises no
           // more flags.  (Asked rarely: hipStreamQuery beside a launch by
           // another thread can report an idle stream.)

@@ -14,6 +14,7 @@
 #include <sstream>
 #include <stdexcept>
 #include <string>
+#include <thread>
 
 namespace kites {
 
@@ -46,6 +47,21 @@ inline void hip_assert(hipError_t err, const char* file, int line) {
     throw std::runtime_error(os.str());
   }
 }
+
+namespace detail {
+
+// One turn of a host thread's wait for a word that the device (or a thread
+// beside it) writes; `turns` so far since the last news.  The first 1,024 spin,
+// some 30 us, longer than most iterations; then the CPU goes to whoever else is
+// ready to run on it.
+inline void wait_turn(unsigned turns) {
+  if (turns < 1024)
+    __builtin_ia32_pause();
+  else
+    std::this_thread::yield();
+}
+
+}  // namespace detail
 
 }  // namespace kites
 

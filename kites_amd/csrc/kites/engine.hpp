@@ -418,7 +418,7 @@ unsigned run_loop(P const& prm, gpu& dev, stream& s, unsigned grid, options cons
       spins = 0;
       since = std::chrono::steady_clock::now();
     }
-    __builtin_ia32_pause();
+    wait_turn(spins);
     // a stream that has failed reports nothing more
     if (++spins % 65536 == 0 &&
         std::chrono::steady_clock::now() - since > std::chrono::seconds(2)) {

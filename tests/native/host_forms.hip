@@ -2,6 +2,10 @@
 #include "forms.hpp"
 #include "native.hpp"
 
+#include <sstream>
+
+#include "host_copy.hpp"
+
 using namespace native;
 
 namespace {
@@ -70,9 +74,32 @@ void functor_mixes() {
   functor_mix<I, N, R, true>();
 }
 
+// CPUs of a container's limit, and a copy's threads within it.
+void cpu_limits() {
+  using namespace kites_capi;
+  std::size_t const none = std::numeric_limits<std::size_t>::max();
+  auto two = [](const char* text) {
+    std::istringstream in(text);
+    return quota_cpus(in, in);
+  };
+  auto split = [](const char* quota, const char* period) {
+    std::istringstream q(quota), p(period);
+    return quota_cpus(q, p);
+  };
+  report("container limits", two("1600000 100000\n") == 16 && two("150000 100000") == 1 &&
+                                 two("20000 100000") == 1 && two("max 100000") == none &&
+                                 two("") == none && two("100000") == none &&
+                                 split("400000\n", "100000\n") == 4 &&
+                                 split("-1\n", "100000\n") == none && split("", "") == none);
+  std::size_t const most = std::min<std::size_t>(container_cpus(), kCopyThreads);
+  report("copy threads", copy_threads(0) == 1 && copy_threads(std::size_t(1) << 20) == 1 &&
+                             copy_threads(std::size_t(1) << 30) <= most);
+}
+
 }  // namespace
 
 int main() {
+  cpu_limits();
   functor_mixes<false, false, false>();
   functor_mixes<false, false, true>();
   functor_mixes<false, true, false>();
