@@ -1188,9 +1188,10 @@ __device__ void run_push_few(P& p, iter_ctx& c, lane_acc& la, step_smem<vT>& sm)
         unsigned const idx = base[own] + (e - excl[own]);
         dst = p.oC[idx];
         vT const cand = edge_value(p.fn, sm.tmp[t], vals[own], p.oE + idx);
-        unsigned const d0 = p.oR[dst], d1 = p.oR[dst + 1];
+        // (in this order: the offsets' difference may be taken, and waited for,
+        // as soon as they are read)
         vT const old = atomic_min_any(p.V + dst, cand);
-        dd = d1 - d0;
+        dd = p.oR[dst + 1] - p.oR[dst];
         if (cand < old && dd) {
           if (is_near(c, cand)) {
             newly = set_bit_now(c.out_bm, dst);
