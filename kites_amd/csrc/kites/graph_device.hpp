@@ -113,7 +113,6 @@ struct workspace {
   // oR (n vertices), computed on `s` the first time and kept.
   const unsigned* maxdeg_of(const unsigned* oR, std::size_t nv, stream& s) {
     if (have_maxdeg) return maxdeg.get_ptr();
-    have_maxdeg = true;
     hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, s.get(), maxdeg.get_ptr(), 1u);
     if (nv) {
       unsigned const blocks = static_cast<unsigned>(std::min<std::size_t>((nv + 1023) / 1024, 512));
@@ -121,6 +120,7 @@ struct workspace {
                          static_cast<unsigned>(nv), maxdeg.get_ptr());
     }
     KITES_HIP_CHECK(hipPeekAtLastError());
+    have_maxdeg = true;
     return maxdeg.get_ptr();
   }
 
