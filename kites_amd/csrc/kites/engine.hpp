@@ -881,6 +881,16 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   }
   param_block<P> const kpb(prm, funcInit, funcCompNbr, funcRed, funcUpd);
   P const& kp = kpb.get();
+  // A call that fails in between (a capture without memory, say) returns when its
+  // launches are done: they still write the progress word and the run state, which
+  // the graph's next run clears from the host and on its stream, and which another
+  // graph's run may share (run states the caller owns).
+  struct drain {
+    hipStream_t s;
+    ~drain() {
+      if (s) (void)hipStreamSynchronize(s);
+    }
+  } unfinished{s.get()};
 
   auto const t0 = std::chrono::steady_clock::now();
   if (st.ev0) KITES_HIP_CHECK(hipEventRecord(st.ev0, s.get()));
@@ -958,6 +968,7 @@ void run_engine(graph_csr_device<vT, eT, vIdxT>& grph, gpu& dev, funcInitT funcI
   }
   if (st.ev1) KITES_HIP_CHECK(hipEventRecord(st.ev1, s.get()));
   s.sync();
+  unfinished.s = nullptr;
   float ms = 0.f;
   if (st.ev0 && st.ev1)
     KITES_HIP_CHECK(hipEventElapsedTime(&ms, st.ev0, st.ev1));
