@@ -29,9 +29,25 @@ __host__ __device__ __forceinline__ volatile T& as_volatile(T& x) {
 // kernel may call it for an edge whose partial is then dropped.  (One that takes
 // the reference's eT* may write through it: each call then stands for one walk
 // of that edge.)  Either way the pointer is the edge's place in the graph's array.
+// Read off the type of its call operator; generic and overloaded functors count
+// as ones that may write.
+template <class R, class C, class A, class B, class E>
+E edge_param(R (C::*)(A, B, E));
+template <class R, class C, class A, class B, class E>
+E edge_param(R (C::*)(A, B, E) const);
+template <class R, class C, class A, class B, class E>
+E edge_param(R (C::*)(A, B, E) noexcept);
+template <class R, class C, class A, class B, class E>
+E edge_param(R (C::*)(A, B, E) const noexcept);
+
+template <class FN, class eT, class = void>
+struct edge_reader : std::false_type {};
+template <class FN, class eT>
+struct edge_reader<FN, eT, std::void_t<decltype(edge_param(&FN::operator()))>>
+    : std::is_same<decltype(edge_param(&FN::operator())), const eT*> {};
+
 template <class FN, class vT, class eT>
-constexpr bool reads_edge = std::is_invocable<FN&, volatile vT&, vT, const eT*>::value ||
-                            std::is_invocable<FN&, vT&, vT, const eT*>::value;
+constexpr bool reads_edge = edge_reader<FN, eT>::value;
 
 // nbrCompF works on its lane's LDS slot (volatile references).
 template <class FN, class vT, class eT>

@@ -96,9 +96,37 @@ void cpu_limits() {
                              copy_threads(std::size_t(1) << 30) <= most);
 }
 
+// Whether a functor may write its edge is read off its signature; a generic one's
+// body is not looked at with a pointer to const (it need not compile with one).
+struct overloaded {
+  __host__ __device__ void operator()(int& part, int src, int* e) const { part = src + *e; }
+  __host__ __device__ void operator()(int& part, int src, float* e) const { part = src + (*e > 0); }
+};
+
+void edge_writers() {
+  using kites::detail::edge_value_at;
+  using kites::detail::reads_edge;
+  auto generic = [] __host__ __device__(auto& part, auto src, auto* e) {
+    *e += 1;
+    part = src + *e;
+  };
+  auto reader = [] __host__ __device__(int& part, int src, const int* e) { part = src + *e; };
+  auto writer = [] __host__ __device__(int& part, int src, int* e) { part = src + *e; };
+  auto counter = [n = 0] __host__ __device__(volatile int& part, int src, int const* e) mutable noexcept {
+    part = src + *e + n;
+  };
+  int slot = 0, edge = 4;
+  edge_value_at(generic, slot, 1, &edge);
+  report("functors that may write the edge",
+         slot == 6 && edge == 5 && !reads_edge<decltype(generic), int, int> &&
+             reads_edge<decltype(reader), int, int> && !reads_edge<decltype(writer), int, int> &&
+             reads_edge<decltype(counter), int, int> && !reads_edge<overloaded, int, int>);
+}
+
 }  // namespace
 
 int main() {
+  edge_writers();
   cpu_limits();
   functor_mixes<false, false, false>();
   functor_mixes<false, false, true>();
