@@ -42,3 +42,9 @@ def test_functor_forms():
 def test_edge_pointer():
     out = _run("edge_pointer")
     assert out.count("ok:") == 10
+
+
+@pytest.mark.gpu
+def test_volatile_sets():
+    out = _run("volatile_sets")
+    assert out.count("ok:") == 2 * (2 * 17 + 2 * 13 + 2 * 2 + 2)
