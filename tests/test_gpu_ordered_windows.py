@@ -26,8 +26,8 @@ def test_list_starts_beside_a_window(at, after):
     R, C, _, oR, oC, _ = h.arrays()
     W = np.float32(1.0) / np.diff(oR.astype(np.int64)).astype(np.float32)[C]
     d = K.DeviceGraph(h)
-    got, info = d.pagerank(damping=0.85, tol=0.0)
+    got, info = d.pagerank(damping=0.85, tol=1e-4)
     exp, it = O.ordered_pagerank(R, C, W, oR, oC, np.ones(n, np.float32), np.ones(n, np.uint8),
-                                 base=np.float32(1.0) - np.float32(0.85), damp=0.85, tol=0.0)
+                                 base=np.float32(1.0) - np.float32(0.85), damp=0.85, tol=1e-4)
     d.close()
     assert info["iterations"] == it and np.array_equal(got.view(np.uint32), exp.view(np.uint32))
