@@ -91,7 +91,7 @@ typedef struct kites_run_opts {
                                runs 4,096) run many per launch in one workgroup (splits of
                                up to twice the limit too); plain and learned
                                schedules of SSSP, BFS, CC and SSSP_WRAP.  0: off.  Above 1:
-                               that out-edge limit (at most 4,096). */
+                               that out-edge limit (values above 4,096 mean 4,096). */
   int32_t small_grid;       /* workgroups of the launches that follow a small push frontier
                                (entries + out-edges <= 2^18; 0 = one per compute unit) */
   int32_t tiny_grid;        /* ... and a tiny one (<= 2^16; 0 = a quarter of small_grid's
@@ -250,7 +250,9 @@ int kites_graph_stats(kites_graph* g, kites_iter_stats* out, uint32_t cap, uint3
  * (Jacobi iterations, a fixed combine order of each vertex's in-edges), so
  * the float result is defined bit for bit.  No counterpart in the reference
  * (its in-place sum would depend on timing, kernels_single_device.cuh:92-132).
- * out: n floats (may be NULL); max_iterations 0 = 10000. */
+ * out: n floats (may be NULL); max_iterations 0 = 10000.  The handle keeps the
+ * n values, the m edge weights and the run state (some 4(2n + m) + m bytes) for
+ * later calls. */
 int kites_pagerank_f32(kites_graph* g, float damping, float tol, uint32_t max_iterations,
                        float* out, kites_run_info* info);
 

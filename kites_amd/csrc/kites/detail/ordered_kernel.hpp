@@ -24,11 +24,11 @@
 // The order fixes only the tree of each 64-edge chunk and the left-to-right
 // fold of a vertex's chunks, so the work is cut by edges, not by vertices
 // (bound: one gather of Vin per in-edge):
-//   * vertices with more than kLight in-edges ("heavy"): one wave per chunk
+//   * vertices with more than 64 in-edges (ordered_shape::light; "heavy"): one wave per chunk
 //     (ordered_heavy_kernel) leaves the chunk's tree in `hsum`; one lane per
 //     vertex folds them in the next launch;
 //   * the others: one wave takes the consecutive vertices whose in-lists start
-//     in one window of kTaskEdges edges, holds all their edges' partials in LDS
+//     in one window of ordered_shape::task_edges edges, holds all their edges' partials in LDS
 //     and runs every vertex's trees at once (a lane's partner l + s belongs to
 //     the same vertex exactly if both carry the same segment start).
 // One wave per vertex, its chunks in sequence and one mark per out-edge, took

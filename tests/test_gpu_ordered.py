@@ -1,7 +1,7 @@
 """Ordered mode at the edges of its work split (detail/ordered_kernel.hpp):
-in-lists around 64 edges (one chunk), 256 (the light limit), 512 (a task
-window) and long ones, in several orders, with vertices without in-edges
-between them; the values and the iteration count must be the oracle's bit for
+in-lists around 64 edges (one chunk, the light limit) and of the other lengths
+up to 512 and beyond, in several orders (so that lists start all over a task's
+window of 448 edges), with vertices without in-edges between them; the values and the iteration count must be the oracle's bit for
 bit (the combine order is defined, so no tolerance)."""
 import numpy as np
 import pytest

@@ -1,8 +1,8 @@
 """The one-workgroup loop for small push frontiers (persist_kernel.hpp).
 
 After a small push frontier the engine's next chunk starts with a launch of
-one workgroup that runs every iteration whose queue fits it (up to 4,096
-entries and 2,048 out-edges by default) before the step launches take over.  The
+one workgroup that runs every iteration whose queue fits it (up to 2,048
+out-edges by default, 4,096 in near-far runs) before the step launches take over.  The
 results must be the oracle's bit for bit, with the loop and without it
 (options persist on and off), on graphs whose runs are long chains of small
 frontiers (grids, paths, a caterpillar whose queue entries have very uneven
